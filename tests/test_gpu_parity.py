@@ -625,3 +625,34 @@ def test_y_line_layouts_against_the_oracle(E, torch_cuda, precision, ny):
         r = O.cpu_projection(c, A, mg, rtol=1e-12)
         mg.close()
         assert relL2(phi, r["phi"], A.fluid_cells) <= 1e-8
+
+
+@pytest.mark.parametrize("dims", [(7, 64, 5), (21, 65, 3), (9, 129, 7), (17, 256, 3), (96, 33, 90), (128, 65, 67),
+                                  (70, 130, 66), (130, 131, 127), (3, 40, 5)])
+def test_y_line_block_layouts(E, torch_cuda, dims):
+    """Every block layout of the segmented y-line step (line_layout: chosen by line
+    length and line count, differently in FP32 and FP64), at odd sizes that leave
+    partial blocks, short last segments and, where the grid holds it, a sphere whose
+    rows take the decoded form.  The mixed and the FP64 solve meet rtol 1e-12, so their
+    phi agree far below 1e-9, and a wrong line solve would not converge alike: the
+    iteration counts differ by at most one."""
+    torch = torch_cuda
+    nx, ny, nz = dims
+    c = (cases.hill_case(nx, ny, nz, h=0.3, beta=2.0, sphere=(0.6, 0.9, 0.0, 0.3), seed=6) if nx * nz > 4000
+         else cases.channel_case(nx, ny, nz, beta=2.5, seed=6))
+    print(f"y-line block layouts: {c.name}", flush=True)
+    fluid = c.fields["nvert"][1:-1, 1:-1, 1:-1] < 0.1
+    outs = []
+    for precision in (1, 0):
+        h = handle_for(E, c, precision=precision, smoother=2, rtol=1e-12)
+        u = torch.from_numpy(np.ascontiguousarray(c.fields["ucont"])).cuda()
+        phi = torch.zeros(c.shape, dtype=torch.float64, device="cuda")
+        p = torch.zeros_like(phi)
+        ucat = torch.zeros(c.shape + (3,), dtype=torch.float64, device="cuda")
+        st = h.project(u, phi, p, ucat, c.dt, c.st, c.coeff, strict=True)
+        h.close()
+        assert st.max_div <= 1e-8
+        outs.append((phi.cpu().numpy()[1:-1, 1:-1, 1:-1][fluid], st.iterations))
+    (a, ia), (b, ib) = outs
+    assert np.linalg.norm(a - b) <= 1e-9 * np.linalg.norm(b)
+    assert abs(ia - ib) <= 1

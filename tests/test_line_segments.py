@@ -1,11 +1,12 @@
-"""The segmented y-line sweeps (line_seg_sweeps in vfs_v3p2_amd/csrc/pp_mg_dev.hpp):
+"""The segmented y-line sweeps (line_step in vfs_v3p2_amd/csrc/pp_line_dev.hpp):
 both Thomas sweeps are affine recurrences, so a line split into S segments, each
-swept from a zero carry with the product of its multipliers kept, chained through
-the segments' carries and re-swept exactly from its carry, solves the same
-tridiagonal system as the sequential sweep.  Checked here in FP64 on diagonally
-dominant systems of 1 to 256 rows for the two layouts the kernels use (16
-segments of up to 16 rows, 32 of up to 8), including lines shorter than the
-segment count (empty segments carry the identity)."""
+swept from a zero carry with the product of its multipliers kept and chained through
+the segments' carries, solves the same tridiagonal system as the sequential sweep.
+`segmented` re-sweeps every segment from its carry; `affine`, the form the kernels
+take, adds the carry times the row's running product.  Checked here in FP64 on
+diagonally dominant systems of 1 to 256 rows for 16 and 32 segments, including lines
+shorter than the segment count (empty segments carry the identity), and the affine
+form's FP32 error against the sequential sweep's."""
 import numpy as np
 import pytest
 
@@ -96,3 +97,58 @@ def test_segmented_sweeps_solve_the_line(ny, segs):
     T = np.diag(b) + np.diag(a[1:], -1) + np.diag(c[:-1], 1)
     assert np.abs(T @ z_seg - r).max() <= 1e-14 * max(1.0, np.abs(r).max())
     assert np.abs(z_seg - z_seq).max() <= 1e-14 * np.abs(z_seq).max()
+
+
+def affine(a, cp, inv, r, S, dt=np.float64):
+    a, cp, inv, r = (v.astype(dt) for v in (a, cp, inv, r))
+    ny = len(r)
+    L = (ny + S - 1) // S
+    rows = [range(s * L, s * L + max(0, min(L, ny - s * L))) for s in range(S)]
+    d, P = np.zeros(ny, dt), np.zeros(ny, dt)
+    ends = []
+    for seg in rows:
+        v, p = dt(0), dt(1)
+        for j in seg:
+            v, p = dt((r[j] - a[j] * v) * inv[j]), dt(p * -(a[j] * inv[j]))
+            d[j], P[j] = v, p
+        ends.append((v, p))
+    c, up = dt(0), np.zeros(ny, dt)
+    for seg, (v, p) in zip(rows, ends):
+        for j in seg:
+            up[j] = d[j] + P[j] * c
+        c = dt(v + p * c)
+    ends = []
+    for seg in rows:
+        v, p = dt(0), dt(1)
+        for j in reversed(seg):
+            v, p = dt(up[j] - cp[j] * v), dt(p * -cp[j])
+            d[j], P[j] = v, p
+        ends.append((v, p))
+    c, z = dt(0), np.zeros(ny, dt)
+    for seg, (v, p) in reversed(list(zip(rows, ends))):
+        for j in seg:
+            z[j] = d[j] + P[j] * c
+        c = dt(v + p * c)
+    return z
+
+
+@pytest.mark.parametrize("segs", [16, 32])
+@pytest.mark.parametrize("ny", [1, 5, 16, 17, 31, 100, 128, 255, 256])
+def test_affine_sweeps_solve_the_line(ny, segs):
+    rng = np.random.default_rng(ny + 1000 * segs)
+    a, c = rng.uniform(-1.0, 0.0, (2, ny))
+    b = 2.05 + rng.uniform(0.0, 0.1, ny)
+    a[0] = c[-1] = 0.0
+    if ny > 8:
+        a[3], b[3], c[3] = 0.0, 1.0, 0.0
+    cp, inv = thomas_factors(a, b, c)
+    r = rng.standard_normal(ny)
+    z_seq = sequential(a, cp, inv, r)
+    scale = np.abs(z_seq).max()
+    assert np.abs(affine(a, cp, inv, r, segs) - z_seq).max() <= 1e-14 * scale
+    # in FP32 every value sees at most one more rounding of a product and a sum per sweep
+    # than in the sequential sweep, whose own error is a few eps on these systems
+    f = np.float32
+    e_seq = np.abs(affine(a, cp, inv, r, 1, f) - z_seq).max() / scale  # one segment: the sequential sweep
+    e_aff = np.abs(affine(a, cp, inv, r, segs, f) - z_seq).max() / scale
+    assert e_aff <= e_seq + 4 * np.finfo(f).eps

@@ -29,6 +29,7 @@
 
 #include "pp_engine.hpp"
 #include "pp_krylov_dev.hpp"
+#include "pp_line_dev.hpp"
 #include "pp_mg_dev.hpp"
 #include "pp_path_dev.hpp"
 
@@ -124,8 +125,8 @@ struct SmoothItem {
   const T* dinv;
   const T* xin;
   T* xout;
-  T* xprev;  // point levels: the previous iterate (read and/or written; may be xout)
-  T* dv;     // y-line levels: the Chebyshev direction
+  T* xprev;  // the previous iterate (may be xout; point levels may write it; y-line levels: null for zero)
+  T* dv;     // power iteration only
   T* out_base;  // non-null: the output is out_base + j * out_stride (the case's Z_j)
   size_t out_stride;
   const T* lfac;  // y-line levels: Thomas factors; scr holds the residual and the forward sweep
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(256) void kb_resid(const SmoothItem<T>* __restrict_
 }
 
 // one Chebyshev step with the y-line preconditioner, one thread per (i, k) line
-template <typename T, bool ZG>
+template <typename T, int MODE>
 __global__ __launch_bounds__(256) void kb_line(const SmoothItem<T>* __restrict__ items,
                                                const uint32_t* __restrict__ start, int nitems, uint32_t total,
                                                const SlotDev* __restrict__ sd) {
@@ -249,19 +250,20 @@ __global__ __launch_bounds__(256) void kb_line(const SmoothItem<T>* __restrict__
     if (!flat_line(I.L.d, t - start[q], i, k)) continue;
     T* xout = I.out_base ? I.out_base + (size_t)st.x * I.out_stride : I.xout;
     const size_t n = I.L.d.n();
-    line_solve_col<T, ZG>(I.L.d, ZG ? I.f : I.scr, I.lfac, I.scr + n, I.xin, xout, I.dv, I.c1, I.c2, i, k);
+    line_solve_col<T, MODE>(I.L.d, MODE == LS_ZERO ? I.f : I.scr, I.lfac, I.scr + n, I.xin, I.xprev, xout, I.c1, I.c2,
+                            i, k);
   }
 }
 
-// the same step with each line split over the waves of a (64, 16) block,
-// line_lanes<T>() consecutive lines (i fastest, then k) per tile, the residual of a step from a
-// non-zero x computed in the same pass; every thread of the block takes part in
-// the barriers of the segmented sweeps, lanes past the last line too
-template <typename T, bool ZG>
-__global__ __launch_bounds__(1024) void kb_line_seg(const SmoothItem<T>* __restrict__ items,
-                                                              const uint32_t* __restrict__ start, int nitems,
-                                                              uint32_t total, const SlotDev* __restrict__ sd) {
-  __shared__ LineSegLds<T> sh;
+// the segmented y-line step (line_step) of layout Y on LANES consecutive lines (i
+// fastest, then k) per tile; every thread of the block takes part in the step's barriers, lanes past the
+// last line too
+template <typename T, typename Y, int MODE>
+__global__ __launch_bounds__(64 * Y::W) void kb_line_step(const SmoothItem<T>* __restrict__ items,
+                                                       const uint32_t* __restrict__ start, int nitems, uint32_t total,
+                                                       const SlotDev* __restrict__ sd) {
+  __shared__ LineLds<T, Y::S, Y::LANES> sh;
+  constexpr int LANES = Y::LANES;
   FOR_TILES(total, t) {
     const uint32_t tw_ = start[nitems + t];
     const int q = (int)(tw_ >> 16);
@@ -269,15 +271,12 @@ __global__ __launch_bounds__(1024) void kb_line_seg(const SmoothItem<T>* __restr
     const SlotDev st = sd[tw_ & 0xffffu];
     if (!st.y) continue;  // the whole block skips the tile
     const uint32_t nx = (uint32_t)I.L.d.nx;
-    const uint32_t e = (t - start[q]) * (uint32_t)line_lanes<T>() + (uint32_t)line_lane<T>();
+    const uint32_t e = (t - start[q]) * (uint32_t)LANES + (threadIdx.x & (uint32_t)(LANES - 1));
     const bool live = e < nx * (uint32_t)I.L.d.nz;
     const int k = live ? (int)(e / nx) : 0;
     const int i = live ? (int)(e - (uint32_t)k * nx) : 0;
     T* xout = I.out_base ? I.out_base + (size_t)st.x * I.out_stride : I.xout;
-    if constexpr (ZG)
-      line_solve_seg<T, true>(I.L.d, live, i, k, I.f, I.lfac, I.xin, xout, I.dv, I.c1, I.c2, sh);
-    else
-      line_step_cell<T>(I.L, live, i, k, I.f, I.lfac, I.xin, xout, I.dv, I.c1, I.c2, sh);
+    line_step<T, Y, MODE>(I.L, live, i, k, I.f, I.lfac, I.xin, I.xprev, xout, I.c1, I.c2, sh);
   }
 }
 
@@ -872,19 +871,27 @@ struct BatchCore {
 
   static uint32_t cell_tiles(const Dims& d) { return (uint32_t)((d.n() + 255) / 256); }
   static uint32_t line_tiles(const Dims& d) { return (uint32_t)(((size_t)d.nx * d.nz + 255) / 256); }
-  static uint32_t seg_line_tiles(const Dims& d) {
-    return (uint32_t)(((size_t)d.nx * d.nz + line_lanes<T>() - 1) / line_lanes<T>());
+  static uint32_t seg_line_tiles(const Dims& d, int layout) {
+    size_t lanes = 1;
+    with_line_layout<T>(layout, [&](auto y) { lanes = decltype(y)::LANES; });
+    return (uint32_t)(((size_t)d.nx * d.nz + lanes - 1) / lanes);
   }
   static bool seg_lines(const Dims& d) { return line_seg_fits<T>(d); }
 
   // Launches of one smoothing step k (0-based) at one depth for a group of
-  // members: point levels fuse the first two steps from a zero start; y-line
-  // levels run a residual launch and a line-solve launch per step (the zero-start
-  // step needs no residual).  cur[] tracks each member's current x buffer.
+  // members: point levels fuse the first two steps from a zero start; y-line levels
+  // run one segmented step per launch layout, or (long lines) a residual launch and a
+  // line-solve launch.  cur[] tracks each member's current x buffer.
   void smoothing_step(int d, int k, bool zero_start, bool final_level0, const std::vector<int>& grp,
                       std::vector<std::vector<T*>>& cur) {
-    std::vector<SmoothItem<T>> pt, rs, lz, lnx, sz, snx;
-    std::vector<uint32_t> npt, nrs, nlz, nlnx, nsz, nsnx;
+    std::vector<SmoothItem<T>> pt, rs, lz, lnx, sg[LINE_LAYOUTS];
+    std::vector<uint32_t> npt, nrs, nlz, nlnx, nsg[LINE_LAYOUTS];
+    int smode = SM_NEXT;
+    size_t lines = 0;  // of the group's y-line levels at this depth
+    for (int q : grp) {
+      auto& L = slots[q].mg->lev[d];
+      if (L.lfac) lines += (size_t)L.d.nx * L.d.nz;
+    }
     int pmode = -1;
     for (int q : grp) {
       auto& L = slots[q].mg->lev[d];
@@ -909,6 +916,7 @@ struct BatchCore {
       it.xin = xin;
       it.xout = xout;
       it.xprev = (mode == SM_NEXT) ? xout : xin;
+      if (line && zero_start && k == 1) it.xprev = nullptr;  // y-line levels start from zero without storing it
       it.dv = L.dv;
       it.out_base = fin ? static_cast<T*>(slots[q].h->Z) : nullptr;
       it.out_stride = L.d.n();
@@ -938,8 +946,10 @@ struct BatchCore {
         it.tx = (uint32_t)(L.d.nx + 63) / 64;
         it.ty = 0;
         if (seg_lines(L.d)) {
-          if (mode == SM_ZERO) { sz.push_back(it); nsz.push_back(seg_line_tiles(L.d)); }
-          else { snx.push_back(it); nsnx.push_back(seg_line_tiles(L.d)); }
+          const int lay = line_layout<T>(L.d.ny, lines);
+          smode = mode;
+          sg[lay].push_back(it);
+          nsg[lay].push_back(seg_line_tiles(L.d, lay));
         } else if (mode == SM_ZERO) {
           lz.push_back(it);
           nlz.push_back(line_tiles(L.d));
@@ -953,8 +963,7 @@ struct BatchCore {
     add_launch_cells(K_RESID, 0, rs);
     add_launch(K_LINE, SM_ZERO, lz, nlz);
     add_launch(K_LINE, SM_NEXT, lnx, nlnx);
-    add_launch(K_LSEG, SM_ZERO, sz, nsz);
-    add_launch(K_LSEG, SM_NEXT, snx, nsnx);
+    for (int y = 0; y < LINE_LAYOUTS; y++) add_launch(K_LSEG, smode + 8 * y, sg[y], nsg[y]);
   }
 
   void build_plan() {
@@ -1224,19 +1233,21 @@ struct BatchCore {
         break;
       case K_LINE:
         if (L.mode == SM_ZERO)
-          kb_line<T, true><<<W, dim3(64, 4, 1), 0, s>>>(static_cast<const SmoothItem<T>*>(L.items), L.start,
-                                                        L.nitems, L.total, sd);
+          kb_line<T, LS_ZERO><<<W, dim3(64, 4, 1), 0, s>>>(static_cast<const SmoothItem<T>*>(L.items), L.start,
+                                                           L.nitems, L.total, sd);
         else
-          kb_line<T, false><<<W, dim3(64, 4, 1), 0, s>>>(static_cast<const SmoothItem<T>*>(L.items), L.start,
-                                                         L.nitems, L.total, sd);
+          kb_line<T, LS_NEXT><<<W, dim3(64, 4, 1), 0, s>>>(static_cast<const SmoothItem<T>*>(L.items), L.start,
+                                                           L.nitems, L.total, sd);
         break;
       case K_LSEG:
-        if (L.mode == SM_ZERO)
-          kb_line_seg<T, true><<<W, dim3(64, 16, 1), 0, s>>>(static_cast<const SmoothItem<T>*>(L.items),
-                                                                    L.start, L.nitems, L.total, sd);
-        else
-          kb_line_seg<T, false><<<W, dim3(64, 16, 1), 0, s>>>(static_cast<const SmoothItem<T>*>(L.items),
-                                                                     L.start, L.nitems, L.total, sd);
+        with_line_layout<T>(L.mode >> 3, [&](auto lay) {
+          using Y = decltype(lay);
+          auto* it = static_cast<const SmoothItem<T>*>(L.items);
+          if ((L.mode & 7) == SM_ZERO)
+            kb_line_step<T, Y, LS_ZERO><<<W, dim3(64, Y::W), 0, s>>>(it, L.start, L.nitems, L.total, sd);
+          else
+            kb_line_step<T, Y, LS_NEXT><<<W, dim3(64, Y::W), 0, s>>>(it, L.start, L.nitems, L.total, sd);
+        });
         break;
       case K_RBLK:
         kb_restrict_blk<T><<<W, dim3(64, 2, 2), 0, s>>>(static_cast<const RestrictItem<T>*>(L.items), L.start,

@@ -314,6 +314,14 @@ static std::unique_ptr<MG<T>> build_mg(vfs_pp_handle* h) {
     if (line) {
       L.lfac = A.alloc<T>(3 * n);
       launch_line_factors<T>(h->s, L.view(), L.lfac);
+      if constexpr (std::is_same<T, float>::value) {
+        if (line_seg_fits<T>(L.d)) {
+          L.pi = A.alloc<u32x2>(n);
+          L.pj = A.alloc<u32x2>(n);
+          L.pk = A.alloc<u32x2>(n);
+          launch_line_pack(h->s, L.view(), L.lfac, L.pi, L.pj, L.pk);
+        }
+      }
     }
     mg->lev.push_back(L);
   }

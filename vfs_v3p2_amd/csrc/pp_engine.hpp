@@ -148,10 +148,12 @@ struct MG : MGBase {
     const uint8_t* cls = nullptr;
     T *f = nullptr, *xa = nullptr, *xb = nullptr, *dv = nullptr, *dinv = nullptr;
     T* lfac = nullptr;  // y-line Thomas factors [a | cp | inv] when line smoothing
+    // y-line levels in FP32: row records of the segmented step
+    u32x2 *pi = nullptr, *pj = nullptr, *pk = nullptr;
     int line = 0;
     std::vector<T> c1, c2;  // Chebyshev coefficients per smoothing step
     double lam = 0.;
-    LevelView<T> view() const { return LevelView<T>{d, g, gh, code, cls, gs}; }
+    LevelView<T> view() const { return LevelView<T>{d, g, gh, code, cls, gs, pi, pj, pk}; }
   };
   std::vector<Lev> lev;
   T* scr = nullptr;
@@ -198,9 +200,11 @@ struct MG : MGBase {
       T* other = (x == L.xa) ? L.xb : L.xa;
       T* xout = other;
       if (last == degree - 1 && final_out) xout = final_out;
-      // point levels: the previous iterate lives in the other buffer (which the next
-      // iterate overwrites); a step from zero leaves its x_prev where x was
+      // the previous iterate lives in the other buffer (which the next iterate
+      // overwrites); a point step from zero leaves its x_prev where x was
       T* xprev = (mode == SM_NEXT) ? other : xin;
+      // y-line levels start from zero without storing it
+      if (L.line && zero_start && k == 1) xprev = nullptr;
       const T c1 = (mode == SM_ZERO || last == 0) ? T(0) : L.c1[last];
       launch_smooth<T>(s, L.view(), L.lfac, mode, L.f, L.dinv, xin, xprev, xout, L.dv, scr, c1, L.c2[last],
                        L.c2[0], mode == SM_FIRST2 ? fdl : nullptr);
@@ -335,6 +339,9 @@ struct MG : MGBase {
       C.dv = dup(L0.dv, n);
       C.dinv = dup(L0.dinv, n);
       C.lfac = dup(L0.lfac, 3 * n);
+      C.pi = dup(L0.pi, n);
+      C.pj = dup(L0.pj, n);
+      C.pk = dup(L0.pk, n);
     }
     for (auto& sc : scrs) sc = tmp.alloc<T>(2 * n);
     auto sweep = [&](int q) {

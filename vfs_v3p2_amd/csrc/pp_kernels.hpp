@@ -173,6 +173,8 @@ void launch_scale_conv(hipStream_t s, size_t n, const double* a, const double* n
                        const TF* dinv = nullptr, TF* fd = nullptr);
 
 // ---- multigrid ---------------------------------------------------------------------
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
 // A multigrid level as the kernels see it.  The levels of the FP32 hierarchy keep
 // their face coefficients in gh as FP16 scaled by a power of two (gh * gs are the
 // coefficients); FP64 levels keep them in g.  FP16 halves the coefficient bytes,
@@ -185,26 +187,36 @@ struct LevelView {
   const uint32_t* code;
   const uint8_t* cls;  // CLS_NONFLUID (transfers) and CLS_INTERIOR (point smoother)
   T gs;
+  // y-line levels of the FP32 hierarchy: the row records of the segmented step (see
+  // pp_line_dev.hpp), 8 bytes per cell each
+  const u32x2 *pi, *pj, *pk;
 };
 
-// Layout of the segmented y-line step (see line_solve_seg): lines per 1024-thread
-// block, segments per line and rows per segment by precision; lines of up to
-// line_segs * line_seg_rows rows take it, longer ones one thread per line.
-template <typename T>
-constexpr int line_lanes() {
-  return sizeof(T) == 4 ? 64 : 32;
-}
-template <typename T>
-constexpr int line_segs() {
-  return 1024 / line_lanes<T>();
-}
-template <typename T>
-constexpr int line_seg_rows() {
-  return sizeof(T) == 4 ? 16 : 8;
-}
+// Lines of up to 256 rows take the segmented y-line step (line_step), longer ones one
+// thread per line.
 template <typename T>
 HD inline bool line_seg_fits(const Dims& d) {
-  return d.ny <= line_segs<T>() * line_seg_rows<T>();
+  return d.ny <= 256;
+}
+// Block layout of the segmented step for lines of ny rows, `lines` of them in the
+// launch (all members of a batched one): an index into line_layouts<T>.  Few lines take
+// narrow blocks of few waves, so that every CU gets some and a block's barriers cost
+// little; many lines take wide ones, whose 256-byte accesses stream from HBM better.
+// The bounds are where the measured step times cross, in us (narrow / middle / wide):
+// FP32 64x64x64 6.4 / 7.2 / 9.5, 256x64x256 37.4 / 37.3 / 41.2, 64x100x64 - / 9.0 / 12.2,
+// 100x110x100 - / 20.5 / 15.8, 64x200x32 10.9 / 18.3 / 20.4, 128x256x64 21.7 / 20.5 / 27.3,
+// 512x256x256 394 / 384 / 375; FP64 64x100x64 15.5 / - / 31.1, 131x77x93 44.0 / - / 28.9,
+// 100x200x100 69.3 / 75.4 / -.
+constexpr int LINE_LAYOUTS = 7;
+template <typename T>
+inline int line_layout(int ny, size_t lines) {
+  if (sizeof(T) == 4) {
+    if (ny <= 64) return lines < 8192 ? 0 : 1;
+    if (ny <= 128) return lines < 8192 ? 2 : 3;
+    return lines < 4096 ? 4 : lines < 16384 ? 5 : 6;
+  }
+  if (ny <= 64) return 0;
+  return ny <= 128 && lines >= 8192 ? 2 : 1;
 }
 
 // Chebyshev smoothing launch modes (see smooth_point_cell); SM_POWER is one step
@@ -220,6 +232,10 @@ void launch_smooth(hipStream_t s, LevelView<T> L, const T* lfac, int mode, const
                    const T* x_old, T* x_prev, T* x_new, T* dv, T* scr, T c1, T c2, T c0, const T* fd = nullptr);
 template <typename T>
 void launch_line_factors(hipStream_t s, LevelView<T> L, T* lfac);
+// the segmented step's row records from the level's FP16 coefficients, class bytes and
+// Thomas factors
+void launch_line_pack(hipStream_t s, const LevelView<float>& L, const float* lfac, u32x2* pi, u32x2* pj,
+                      u32x2* pk);
 // streaming floor of a point sweep: reads every array the sweep reads once per
 // cell (class byte, nine coefficient arrays, f, x, the previous iterate) and
 // writes one, with no stencil

@@ -11,7 +11,7 @@
 // next to coarse IB cells and at non-periodic walls, periodic axes wrap.
 #include <algorithm>
 
-#include "pp_mg_dev.hpp"
+#include "pp_line_dev.hpp"
 
 namespace pp {
 
@@ -60,36 +60,41 @@ __global__ __launch_bounds__(256) void k_resid(LevelView<T> L, const T* __restri
   resid_cell(L, f, x, r, i, j, k);
 }
 
-template <typename T, bool ZG>
+template <typename T, int MODE>
 __global__ __launch_bounds__(256) void k_line_solve(Dims d, const T* __restrict__ r, const T* __restrict__ lfac,
                                                     T* __restrict__ tmp, const T* __restrict__ x_old,
-                                                    T* __restrict__ x_new, T* __restrict__ dv, T c1, T c2) {
+                                                    const T* x_prev, T* x_new, T c1, T c2) {
   const int i = blockIdx.x * 64 + threadIdx.x, k = blockIdx.y * 4 + threadIdx.y;
   if (i >= d.nx || k >= d.nz) return;
-  line_solve_col<T, ZG>(d, r, lfac, tmp, x_old, x_new, dv, c1, c2, i, k);
+  line_solve_col<T, MODE>(d, r, lfac, tmp, x_old, x_prev, x_new, c1, c2, i, k);
 }
 
-// line_lanes<T>() lines (i = line_lanes<T>() blockIdx.x + line_lane<T>(), k =
-// blockIdx.y) per (64, 16) block
-template <typename T, bool ZG>
-__global__ __launch_bounds__(1024) void k_line_seg(Dims d, const T* __restrict__ r,
-                                                             const T* __restrict__ lfac,
-                                                             const T* __restrict__ x_old, T* __restrict__ x_new,
-                                                             T* __restrict__ dv, T c1, T c2) {
-  __shared__ LineSegLds<T> sh;
-  const int i = blockIdx.x * line_lanes<T>() + line_lane<T>(), k = blockIdx.y;
-  line_solve_seg<T, ZG>(d, i < d.nx, i, k, r, lfac, x_old, x_new, dv, c1, c2, sh);
+// the segmented y-line step (line_step): LANES consecutive lines (i fastest, then k)
+// per (64, W) block of layout Y, blocks in XCD order so that lines adjacent in k share an L2
+template <typename T, typename Y, int MODE>
+__global__ __launch_bounds__(64 * Y::W) void k_line_step(LevelView<T> L, const T* __restrict__ f,
+                                                      const T* __restrict__ lfac, const T* __restrict__ x_old,
+                                                      const T* x_prev, T* x_new, T c1, T c2) {
+  __shared__ LineLds<T, Y::S, Y::LANES> sh;
+  constexpr int LANES = Y::LANES;
+  const uint32_t nx = (uint32_t)L.d.nx;
+  const uint32_t e = xcd_block().x * (uint32_t)LANES + (threadIdx.x & (uint32_t)(LANES - 1));
+  const bool live = e < nx * (uint32_t)L.d.nz;
+  const int k = live ? (int)(e / nx) : 0;
+  const int i = live ? (int)(e - (uint32_t)k * nx) : 0;
+  line_step<T, Y, MODE>(L, live, i, k, f, lfac, x_old, x_prev, x_new, c1, c2, sh);
 }
 
-// residual and line step in one pass, same block layout as k_line_seg
-template <typename T>
-__global__ __launch_bounds__(1024) void k_line_fused(LevelView<T> L, const T* __restrict__ f,
-                                                               const T* __restrict__ lfac,
-                                                               const T* __restrict__ x_old, T* __restrict__ x_new,
-                                                               T* __restrict__ dv, T c1, T c2) {
-  __shared__ LineSegLds<T> sh;
-  const int i = blockIdx.x * line_lanes<T>() + line_lane<T>(), k = blockIdx.y;
-  line_step_cell<T>(L, i < L.d.nx, i, k, f, lfac, x_old, x_new, dv, c1, c2, sh);
+__global__ __launch_bounds__(256) void k_line_pack(size_t n, const _Float16* __restrict__ g,
+                                                   const uint8_t* __restrict__ cls, const float* __restrict__ inv,
+                                                   u32x2* __restrict__ pi, u32x2* __restrict__ pj,
+                                                   u32x2* __restrict__ pk) {
+  const size_t c = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (c >= n) return;
+  auto half = [&](int a) -> uint32_t { return __builtin_bit_cast(uint16_t, g[(size_t)a * n + c]); };
+  pi[c] = u32x2{half(0) | half(1) << 16, half(2) | (uint32_t)cls[c] << 16};
+  pj[c] = u32x2{half(4) | half(5) << 16, __builtin_bit_cast(uint32_t, inv[c])};
+  pk[c] = u32x2{half(6) | half(7) << 16, half(8) | half(3) << 16};
 }
 
 // HALF: the coefficients are FP16 (gh), else T (g)
@@ -577,6 +582,21 @@ inline unsigned nb1(size_t n) { return (unsigned)((n + 255) / 256); }
 }  // namespace
 
 template <typename T>
+static void launch_line_step(hipStream_t s, const LevelView<T>& L, int mode, const T* f, const T* lfac,
+                             const T* x_old, const T* x_prev, T* x_new, T c1, T c2) {
+  with_line_layout<T>(line_layout<T>(L.d.ny, (size_t)L.d.nx * L.d.nz), [&](auto lay) {
+    using Y = decltype(lay);
+    const dim3 gr((unsigned)(((size_t)L.d.nx * L.d.nz + Y::LANES - 1) / Y::LANES)), bl(64, Y::W);
+    if (mode == LS_ZERO)
+      k_line_step<T, Y, LS_ZERO><<<gr, bl, 0, s>>>(L, f, lfac, x_old, x_prev, x_new, c1, c2);
+    else if (mode == LS_POWER)
+      k_line_step<T, Y, LS_POWER><<<gr, bl, 0, s>>>(L, f, lfac, x_old, x_prev, x_new, c1, c2);
+    else
+      k_line_step<T, Y, LS_NEXT><<<gr, bl, 0, s>>>(L, f, lfac, x_old, x_prev, x_new, c1, c2);
+  });
+}
+
+template <typename T>
 void launch_smooth(hipStream_t s, LevelView<T> L, const T* lfac, int mode, const T* f, const T* dinv,
                    const T* x_old, T* x_prev, T* x_new, T* dv, T* scr, T c1, T c2, T c0, const T* fd) {
   if (lfac) {
@@ -585,16 +605,19 @@ void launch_smooth(hipStream_t s, LevelView<T> L, const T* lfac, int mode, const
     if (mode == SM_FIRST2) throw StatusError(1, "the line smoother has no fused first-two-steps mode");
     // lines of up to 256 rows are split over the waves of a block
     const bool seg = line_seg_fits<T>(L.d);
-    const dim3 sgrid((L.d.nx + line_lanes<T>() - 1) / line_lanes<T>(), L.d.nz), sblk(64, 16);
-    if (mode == SM_ZERO) {
-      if (seg) k_line_seg<T, true><<<sgrid, sblk, 0, s>>>(L.d, f, lfac, x_old, x_new, dv, c1, c2);
-      else k_line_solve<T, true><<<line_grid(L.d), kBlk, 0, s>>>(L.d, f, lfac, scr + n, x_old, x_new, dv, c1, c2);
-    } else if (seg) {
-      k_line_fused<T><<<sgrid, sblk, 0, s>>>(L, f, lfac, x_old, x_new, dv, c1, c2);
+    if (seg) {
+      if (mode == SM_POWER) launch_line_step<T>(s, L, LS_POWER, f, lfac, x_old, nullptr, dv, c1, c2);
+      else launch_line_step<T>(s, L, mode == SM_ZERO ? LS_ZERO : LS_NEXT, f, lfac, x_old, x_prev, x_new, c1, c2);
+    } else if (mode == SM_ZERO) {
+      k_line_solve<T, LS_ZERO><<<line_grid(L.d), kBlk, 0, s>>>(L.d, f, lfac, scr + n, x_old, x_prev, x_new, c1, c2);
     } else {
       k_resid<T><<<cell_grid(L.d), kBlk, 0, s>>>(L, f, x_old, scr);
       HIPCHECK(hipGetLastError());
-      k_line_solve<T, false><<<line_grid(L.d), kBlk, 0, s>>>(L.d, scr, lfac, scr + n, x_old, x_new, dv, c1, c2);
+      if (mode == SM_POWER)
+        k_line_solve<T, LS_POWER><<<line_grid(L.d), kBlk, 0, s>>>(L.d, scr, lfac, scr + n, x_old, nullptr, dv, c1, c2);
+      else
+        k_line_solve<T, LS_NEXT><<<line_grid(L.d), kBlk, 0, s>>>(L.d, scr, lfac, scr + n, x_old, x_prev, x_new, c1,
+                                                                 c2);
     }
   } else {
     switch (mode) {
@@ -635,6 +658,13 @@ void launch_line_factors(hipStream_t s, LevelView<T> L, T* lfac) {
   k_line_rows<T><<<cell_grid(L.d), kBlk, 0, s>>>(L, lfac);
   HIPCHECK(hipGetLastError());
   k_line_factors<T><<<line_grid(L.d), kBlk, 0, s>>>(L.d, lfac);
+  HIPCHECK(hipGetLastError());
+}
+
+void launch_line_pack(hipStream_t s, const LevelView<float>& L, const float* lfac, u32x2* pi, u32x2* pj,
+                      u32x2* pk) {
+  const size_t n = L.d.n();
+  k_line_pack<<<nb1(n), 256, 0, s>>>(n, L.gh, L.cls, lfac + 2 * n, pi, pj, pk);
   HIPCHECK(hipGetLastError());
 }
 

@@ -254,17 +254,21 @@ __device__ __forceinline__ void resid_cell(const LevelView<T>& L, const T* __res
   resid_body(L, L.g, false, f, x, r, i, j, k);
 }
 
+// what a y-line step computes: LS_ZERO the step from x = 0 (r = f); LS_NEXT a step from
+// x_old; LS_POWER z alone, to x_new (the power iteration)
+enum { LS_NEXT = 0, LS_ZERO = 1, LS_POWER = 2 };
+
 // One Chebyshev step preconditioned by the y-line tridiagonal part T of A on the
-// line (i, k): z = T^-1 r with the precomputed factors (forward sweep parked in
-// tmp), d = c1 d + c2 z, x_new = x_old + d.  ZG: from x = 0 with r = f.
+// line (i, k), in three-term form: z = T^-1 r with the precomputed factors (forward
+// sweep parked in tmp), x_new = x + c1 (x - x_prev) + c2 z (x_prev null: zero; x_new may
+// be x_prev's buffer).  For lines too long for the segmented step (pp_line_dev.hpp).
 // The line is walked in chunks of LC rows whose inputs are loaded into registers
 // first (independent loads in flight together), then the recurrence runs on them:
 // the sequential sweep is otherwise bound by one load latency per row.
-template <typename T, bool ZG>
+template <typename T, int MODE>
 __device__ __forceinline__ void line_solve_col(const Dims& d, const T* __restrict__ r, const T* __restrict__ lfac,
-                                               T* __restrict__ tmp, const T* __restrict__ x_old,
-                                               T* __restrict__ x_new, T* __restrict__ dv, T c1, T c2, int i,
-                                               int k) {
+                                               T* __restrict__ tmp, const T* __restrict__ x_old, const T* x_prev,
+                                               T* x_new, T c1, T c2, int i, int k) {
   constexpr int LC = 16;
   const size_t n = d.n();
   const T* __restrict__ la = lfac;
@@ -293,17 +297,17 @@ __device__ __forceinline__ void line_solve_col(const Dims& d, const T* __restric
     }
   }
   T znext = T(0);
-  const bool rd = !ZG && c1 != T(0);
+  const bool rd = MODE == LS_NEXT && c1 != T(0) && x_prev;
   for (int j1 = ny - 1; j1 >= 0; j1 -= LC) {
-    T tt[LC], pp[LC], dd[LC], xo[LC];
+    T tt[LC], pp[LC], xq[LC], xo[LC];
 #pragma unroll
     for (int q = 0; q < LC; q++) {
       const int j = j1 - q >= 0 ? j1 - q : 0;
       const size_t c = c0 + (size_t)j * sy;
       tt[q] = tmp[c];
       pp[q] = lcp[c];
-      dd[q] = rd ? dv[c] : T(0);
-      xo[q] = ZG ? T(0) : x_old[c];
+      xq[q] = rd ? x_prev[c] : T(0);
+      xo[q] = MODE == LS_NEXT ? x_old[c] : T(0);
     }
 #pragma unroll
     for (int q = 0; q < LC; q++) {
@@ -311,276 +315,10 @@ __device__ __forceinline__ void line_solve_col(const Dims& d, const T* __restric
         const size_t c = c0 + (size_t)(j1 - q) * sy;
         const T z = tt[q] - pp[q] * znext;
         znext = z;
-        const T dn = c1 * dd[q] + c2 * z;
-        dv[c] = dn;
-        x_new[c] = xo[q] + dn;
+        x_new[c] = MODE == LS_POWER ? z : (MODE == LS_ZERO ? c2 * z : xo[q] + (c1 * (xo[q] - xq[q]) + c2 * z));
       }
     }
   }
-}
-
-// The same Chebyshev step with each line split into segments of a few rows held
-// in registers.  A (64, 16) block of 1024 threads holds line_lanes<T>() lines:
-// in FP32 64 lines of 16 segments of up to 16 rows (wave w takes segment w of
-// every line), in FP64 32 lines of 32 segments of up to 8 rows (lanes 0-31 of
-// wave w take segment 2w, lanes 32-63 segment 2w + 1), so lines of up to 256 rows
-// fit either way within the registers a 1024-thread block allows.  Lines of up
-// to 256 rows keep 16 or 32 times more lanes busy than one thread per line, and
-// the forward sweep stays in registers instead of going through memory.  Both
-// sweeps are affine recurrences, d_j = (r_j - a_j d_{j-1}) inv_j and
-// z_j = d_j - cp_j z_{j+1}; each segment first runs its sweep from a zero carry,
-// keeping the product of its multipliers, the carries into every segment follow
-// from one pass over the segments of a line (LDS), and each segment then reruns
-// the recurrence exactly from its carry.  Every thread of the block must call it
-// (block barriers); lanes without a line pass live = false.
-// (line_lanes, line_segs, line_seg_rows and line_seg_fits: pp_kernels.hpp)
-// this thread's line within the block and its segment
-template <typename T>
-__device__ __forceinline__ int line_lane() {
-  return (int)(threadIdx.x & (line_lanes<T>() - 1));
-}
-template <typename T>
-__device__ __forceinline__ int line_seg() {
-  return (int)(threadIdx.y * (64 / line_lanes<T>()) + threadIdx.x / line_lanes<T>());
-}
-template <typename T>
-struct LineSegLds {
-  T part[2][line_segs<T>()][line_lanes<T>()];  // a segment's zero-carry end value and multiplier product
-  T carry[line_segs<T>()][line_lanes<T>()];    // carry into each segment
-};
-
-// The two segmented sweeps of one Chebyshev step: rr holds the segment's nr rows
-// of r (rows j0 .. j0 + nr - 1 of the line whose row j0 is cell c0).
-template <typename T, bool ZG>
-__device__ __forceinline__ void line_seg_sweeps(const Dims& d, size_t c0, int nr,
-                                                const T (&rr)[line_seg_rows<T>()], const T* __restrict__ lfac,
-                                                const T* __restrict__ x_old, T* __restrict__ x_new,
-                                                T* __restrict__ dv, T c1, T c2, LineSegLds<T>& sh) {
-  constexpr int LM = line_seg_rows<T>();
-  const int lane = line_lane<T>(), s = line_seg<T>();
-  const size_t n = d.n();
-  const size_t sy = (size_t)d.nx;
-  const T* __restrict__ la = lfac;
-  const T* __restrict__ lcp = lfac + n;
-  const T* __restrict__ linv = lfac + 2 * n;
-  T aa[LM], vv[LM];
-#pragma unroll
-  for (int q = 0; q < LM; q++) {
-    aa[q] = vv[q] = T(0);
-    if (q < nr) {
-      const size_t c = c0 + (size_t)q * sy;
-      aa[q] = la[c];
-      vv[q] = linv[c];
-    }
-  }
-  // forward sweep from a zero carry: end value and product of the multipliers
-  T dl = T(0), prod = T(1);
-#pragma unroll
-  for (int q = 0; q < LM; q++)
-    if (q < nr) {
-      dl = (rr[q] - aa[q] * dl) * vv[q];
-      prod = prod * -(aa[q] * vv[q]);
-    }
-  sh.part[0][s][lane] = dl;
-  sh.part[1][s][lane] = prod;
-  __syncthreads();
-  if (s == 0) {
-    T c = T(0);
-    for (int t = 0; t < line_segs<T>(); t++) {
-      sh.carry[t][lane] = c;
-      c = sh.part[0][t][lane] + sh.part[1][t][lane] * c;
-    }
-  }
-  __syncthreads();
-  T dd[LM];
-  T dprev = sh.carry[s][lane];
-#pragma unroll
-  for (int q = 0; q < LM; q++) {
-    dd[q] = T(0);
-    if (q < nr) {
-      dprev = (rr[q] - aa[q] * dprev) * vv[q];
-      dd[q] = dprev;
-    }
-  }
-  // backward sweep
-  const bool rd = !ZG && c1 != T(0);
-  T pp[LM], dvo[LM], xo[LM];
-#pragma unroll
-  for (int q = 0; q < LM; q++) {
-    pp[q] = dvo[q] = xo[q] = T(0);
-    if (q < nr) {
-      const size_t c = c0 + (size_t)q * sy;
-      pp[q] = lcp[c];
-      if (rd) dvo[q] = dv[c];
-      if (!ZG) xo[q] = x_old[c];
-    }
-  }
-  T zl = T(0);
-  prod = T(1);
-#pragma unroll
-  for (int q = LM - 1; q >= 0; q--)
-    if (q < nr) {
-      zl = dd[q] - pp[q] * zl;
-      prod = prod * -pp[q];
-    }
-  __syncthreads();  // every thread has read its forward carry
-  sh.part[0][s][lane] = zl;
-  sh.part[1][s][lane] = prod;
-  __syncthreads();
-  if (s == 0) {
-    T c = T(0);
-    for (int t = line_segs<T>() - 1; t >= 0; t--) {
-      sh.carry[t][lane] = c;
-      c = sh.part[0][t][lane] + sh.part[1][t][lane] * c;
-    }
-  }
-  __syncthreads();
-  T znext = sh.carry[s][lane];
-#pragma unroll
-  for (int q = LM - 1; q >= 0; q--)
-    if (q < nr) {
-      const size_t c = c0 + (size_t)q * sy;
-      const T z = dd[q] - pp[q] * znext;
-      znext = z;
-      const T dn = c1 * dvo[q] + c2 * z;
-      dv[c] = dn;
-      x_new[c] = xo[q] + dn;
-    }
-  __syncthreads();  // the LDS is free for the block's next tile
-}
-
-// rows of this thread's segment: first row j0, count nr (0 for a lane without a line)
-template <typename T>
-__device__ __forceinline__ void line_seg_rows_of(const Dims& d, bool live, int& j0, int& nr) {
-  const int L = (d.ny + line_segs<T>() - 1) / line_segs<T>();
-  j0 = line_seg<T>() * L;
-  nr = live ? max(0, min(L, d.ny - j0)) : 0;
-}
-
-template <typename T, bool ZG>
-__device__ __forceinline__ void line_solve_seg(const Dims& d, bool live, int i, int k, const T* __restrict__ r,
-                                               const T* __restrict__ lfac, const T* __restrict__ x_old,
-                                               T* __restrict__ x_new, T* __restrict__ dv, T c1, T c2,
-                                               LineSegLds<T>& sh) {
-  constexpr int LM = line_seg_rows<T>();
-  int j0, nr;
-  line_seg_rows_of<T>(d, live, j0, nr);
-  const size_t sy = (size_t)d.nx;
-  const size_t c0 = live ? d.idx(i, j0 < d.ny ? j0 : 0, k) : 0;
-  T rr[LM];
-#pragma unroll
-  for (int q = 0; q < LM; q++) rr[q] = q < nr ? r[c0 + (size_t)q * sy] : T(0);
-  line_seg_sweeps<T, ZG>(d, c0, nr, rr, lfac, x_old, x_new, dv, c1, c2, sh);
-}
-
-// One Chebyshev step (from a non-zero x) with the y-line preconditioner and the
-// residual r = f - A x computed in the same pass: each thread walks its segment's
-// rows, keeping the stencil's values of x in the five columns (i, k), (i +- 1, k),
-// (i, k +- 1) for the rows below, at and above the current one, so a row loads
-// five values of x for the row above plus the four (i +- 1, k +- 1) values of its
-// own row (9 instead of 19), and its lower j-face coefficients are the row below's
-// upper ones.  The row's stencil values and coefficients are the ones the residual
-// kernel reads, and its form is voted over the wave's 64 lines at that row.
-template <typename T, typename TG>
-__device__ __forceinline__ void line_step_fused(const LevelView<T>& L, const TG* __restrict__ g, bool scaled, bool live,
-                                                int i, int k, const T* __restrict__ f, const T* __restrict__ lfac,
-                                                const T* __restrict__ x_old, T* __restrict__ x_new,
-                                                T* __restrict__ dv, T c1, T c2, LineSegLds<T>& sh) {
-  constexpr int LM = line_seg_rows<T>();
-  const Dims& d = L.d;
-  int j0, nr;
-  line_seg_rows_of<T>(d, live, j0, nr);
-  const uint32_t nx = (uint32_t)d.nx, plane = (uint32_t)d.nx * (uint32_t)d.ny;
-  const size_t n = d.n();
-  const int ii = live ? i : 0, kk = live ? k : 0;
-  const uint32_t ip = (uint32_t)wrap_p(ii, d.nx, d.per[0]), im = (uint32_t)wrap_m(ii, d.nx, d.per[0]);
-  const uint32_t kp = (uint32_t)wrap_p(kk, d.nz, d.per[2]) * plane, km = (uint32_t)wrap_m(kk, d.nz, d.per[2]) * plane;
-  const uint32_t ic = (uint32_t)ii, kc = (uint32_t)kk * plane;
-  // column bases (cell index of row 0) of the marched columns C, E, W, T, B and of
-  // the four corner columns read at the row itself
-  const uint32_t col[5] = {ic + kc, ip + kc, im + kc, ic + kp, ic + km};
-  const uint32_t cor[4] = {ip + kp, ip + km, im + kp, im + km};  // TE, BE, TW, BW
-  const int jr = j0 < d.ny ? j0 : 0;
-  const uint32_t rowm0 = (uint32_t)wrap_m(jr, d.ny, d.per[1]) * nx;
-  T xm[5], x0[5];
-#pragma unroll
-  for (int a = 0; a < 5; a++) {
-    xm[a] = nr > 0 ? (T)ld_at(x_old, col[a] + rowm0) : T(0);
-    x0[a] = nr > 0 ? (T)ld_at(x_old, col[a] + (uint32_t)jr * nx) : T(0);
-  }
-  // upper j-face coefficients of the row below the segment
-  TG gs_prev[3];
-#pragma unroll
-  for (int e = 0; e < 3; e++) gs_prev[e] = nr > 0 ? ld_at(g + (size_t)(3 + e) * n, ic + kc + rowm0) : TG(0);
-  T rr[LM];
-#pragma unroll
-  for (int q = 0; q < LM; q++) {
-    rr[q] = T(0);
-    if (q < nr) {
-      const int j = j0 + q;
-      const uint32_t rj = (uint32_t)j * nx, rp = (uint32_t)wrap_p(j, d.ny, d.per[1]) * nx;
-      const uint32_t c = ic + kc + rj;
-      const uint8_t cl = L.cls[c];
-      const T fc = f[c];
-      T xp_[5];
-#pragma unroll
-      for (int a = 0; a < 5; a++) xp_[a] = (T)ld_at(x_old, col[a] + rp);
-      T xv[19];
-      xv[CP] = x0[0]; xv[NP] = xp_[0]; xv[SP] = xm[0];
-      xv[EP] = x0[1]; xv[NE] = xp_[1]; xv[SE] = xm[1];
-      xv[WP] = x0[2]; xv[NW] = xp_[2]; xv[SW] = xm[2];
-      xv[TP] = x0[3]; xv[TN] = xp_[3]; xv[TS] = xm[3];
-      xv[BP] = x0[4]; xv[BN] = xp_[4]; xv[BS] = xm[4];
-      xv[TE] = (T)ld_at(x_old, cor[0] + rj);
-      xv[BE] = (T)ld_at(x_old, cor[1] + rj);
-      xv[TW] = (T)ld_at(x_old, cor[2] + rj);
-      xv[BW] = (T)ld_at(x_old, cor[3] + rj);
-      RowCoef<TG> rc;
-#pragma unroll
-      for (int e = 0; e < 3; e++) {
-        rc.v[0][e] = ld_at(g + (size_t)e * n, c);
-        rc.v[1][e] = ld_at(g + (size_t)e * n, im + kc + rj);
-        rc.v[2][e] = ld_at(g + (size_t)(3 + e) * n, c);
-        rc.v[3][e] = gs_prev[e];
-        rc.v[4][e] = ld_at(g + (size_t)(6 + e) * n, c);
-        rc.v[5][e] = ld_at(g + (size_t)(6 + e) * n, ic + km + rj);
-      }
-      T ax, dg;
-      bool row = true;
-      if (__all((cl & CLS_INTERIOR) != 0)) {
-        flux_row_v<X_CENTRAL>(rc, CODE_INTERIOR, xv, ax, dg);
-      } else {
-        const uint32_t cd = L.code[c];
-        flux_row_v<-1>(rc, cd, xv, ax, dg);
-        row = (cd & ROW_BIT) != 0;
-      }
-      if (scaled) ax *= L.gs;
-      rr[q] = row ? fc - ax : T(0);
-#pragma unroll
-      for (int a = 0; a < 5; a++) {
-        xm[a] = x0[a];
-        x0[a] = xp_[a];
-      }
-#pragma unroll
-      for (int e = 0; e < 3; e++) gs_prev[e] = rc.v[2][e];
-    }
-  }
-  const size_t c0 = nr > 0 ? d.idx(ii, j0, kk) : 0;
-  line_seg_sweeps<T, false>(d, c0, nr, rr, lfac, x_old, x_new, dv, c1, c2, sh);
-}
-
-template <typename T>
-__device__ __forceinline__ void line_step_cell(const LevelView<T>& L, bool live, int i, int k,
-                                               const T* __restrict__ f, const T* __restrict__ lfac,
-                                               const T* __restrict__ x_old, T* __restrict__ x_new,
-                                               T* __restrict__ dv, T c1, T c2, LineSegLds<T>& sh) {
-  if constexpr (std::is_same<T, float>::value) {
-    if (L.gh) {
-      line_step_fused(L, L.gh, true, live, i, k, f, lfac, x_old, x_new, dv, c1, c2, sh);
-      return;
-    }
-  }
-  line_step_fused(L, L.g, false, live, i, k, f, lfac, x_old, x_new, dv, c1, c2, sh);
 }
 
 // fc[C] = sum over fluid children of (f - A x); zero on coarse IB cells.  Any
