@@ -350,3 +350,26 @@ def test_coarse_inverse_matches_lapack(E, name, coarse_max, precision):
     assert np.abs(ce - ref).max() <= tol * scale
     # the system is not trivial: off-diagonal coupling is present
     assert np.abs(ref - np.diag(np.diag(ref))).max() > 1e-3 * scale
+
+
+@pytest.mark.parametrize("dims,coarse_max", [((3, 3, 3), 512), ((4, 2, 4), 512), ((3, 7, 3), 512), ((8, 8, 8), 512),
+                                             ((9, 9, 9), 1000), ((16, 8, 8), 1024)])
+def test_dense_level_alone(E, dims, coarse_max):
+    """A grid that is its own coarsest level: the V-cycle is the dense solve, so the first
+    Krylov step lands on the solution (to the FP32 inverse's rounding in the mixed form,
+    at most three steps).  Sizes around one row block and one batch of columns."""
+    import torch
+
+    nx, ny, nz = dims
+    c = cases.channel_case(nx, ny, nz, beta=1.5, seed=1)
+    for precision, most in ((0, 2), (1, 4)):
+        h = handle(E, c, precision=precision, coarse_max=coarse_max, rtol=1e-12)
+        assert len(h.export_levels(rows=False)) == 1
+        u = torch.from_numpy(np.ascontiguousarray(c.fields["ucont"])).cuda()
+        phi = torch.zeros(c.shape, dtype=torch.float64, device="cuda")
+        p = torch.zeros_like(phi)
+        ucat = torch.zeros(c.shape + (3,), dtype=torch.float64, device="cuda")
+        st = h.project(u, phi, p, ucat, c.dt, c.st, c.coeff, strict=True)
+        h.close()
+        print(f"dense level {dims} precision {precision}: {st.iterations} iterations", flush=True)
+        assert st.iterations <= most and st.max_div <= 1e-8

@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256) void kb_dense(const DenseItem<T>* __restrict__
                                                 const uint32_t* __restrict__ start, int nitems, uint32_t total,
                                                 const SlotDev* __restrict__ sd) {
   __shared__ T fs[1024];
-  __shared__ T part[4][64];
+  __shared__ T part[8][DENSE_ROWS];
   FOR_TILES(total, t) {
     const uint32_t tw_ = start[nitems + t];
     const int q = (int)(tw_ >> 16);
@@ -1057,7 +1057,7 @@ struct BatchCore {
           }
           cur[q][d] = L.xa;
           items.push_back(it);
-          nt.push_back((uint32_t)(it.n + 63) / 64);
+          nt.push_back((uint32_t)(it.n + DENSE_ROWS - 1) / DENSE_ROWS);
         }
         add_launch(K_DENSE, 0, items, nt);
       }

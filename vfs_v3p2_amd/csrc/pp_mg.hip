@@ -146,7 +146,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_dense_solve(int n, const T* __restrict__ cinv, const T* __restrict__ f,
                                                      T* __restrict__ x) {
   __shared__ T fs[1024];
-  __shared__ T part[4][64];
+  __shared__ T part[8][DENSE_ROWS];
   dense_rows(n, cinv, f, x, (int)blockIdx.x, fs, part);
 }
 
@@ -697,7 +697,7 @@ void launch_prolong_add(hipStream_t s, LevelView<T> F, Dims dc, const uint8_t* c
 template <typename T>
 void launch_dense_solve(hipStream_t s, int n, const T* cinv, const T* f, T* x) {
   if (n > 1024) throw StatusError(1, "coarsest level larger than 1024 cells");
-  k_dense_solve<T><<<(n + 63) / 64, 256, 0, s>>>(n, cinv, f, x);
+  k_dense_solve<T><<<(n + DENSE_ROWS - 1) / DENSE_ROWS, 256, 0, s>>>(n, cinv, f, x);
   HIPCHECK(hipGetLastError());
 }
 
