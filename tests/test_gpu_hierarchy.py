@@ -352,6 +352,27 @@ def test_coarse_inverse_matches_lapack(E, name, coarse_max, precision):
     assert np.abs(ref - np.diag(np.diag(ref))).max() > 1e-3 * scale
 
 
+@pytest.mark.parametrize("dims,coarse_max", [((8, 4, 3), 96), ((4, 4, 7), 112), ((9, 9, 9), 1000), ((16, 8, 8), 1024)])
+def test_coarse_inverse_panels(E, dims, coarse_max):
+    """The panelled Gauss-Jordan where it can go wrong: the smallest system the device
+    takes (97 rows, one column in the last panel), a full last panel's edge (113), an odd
+    size over two row tiles (730) and more rows than threads (1025).  The inverse of the
+    whole grid's bordered system against LAPACK, to 1e-9 of its largest entry (measured:
+    3e-12 for systems of this kind)."""
+    nx, ny, nz = dims
+    c = cases.channel_case(nx, ny, nz, beta=1.5, seed=1)
+    A = O.Assembled(c, drop=False)
+    h = handle(E, c, precision=0, coarse_max=coarse_max)
+    levels = h.export_levels(rows=False)
+    ce = h.export_coarse_inverse()
+    h.close()
+    assert len(levels) == 1
+    ref, N = _bordered_inverse(*_oracle_coarsest(c, A, levels), c.per)
+    print(f"coarse inverse panels {dims}: bordered {N}", flush=True)
+    assert N == nx * ny * nz + 1
+    assert np.abs(ce - ref).max() <= 1e-9 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("dims,coarse_max", [((3, 3, 3), 512), ((4, 2, 4), 512), ((3, 7, 3), 512), ((8, 8, 8), 512),
                                              ((9, 9, 9), 1000), ((16, 8, 8), 1024)])
 def test_dense_level_alone(E, dims, coarse_max):

@@ -83,11 +83,9 @@ static std::vector<double> coarse_bordered(const CoarseRows& L, int* ncomp_out) 
   return B;
 }
 
-// The same elimination as launch_gj_step (partial pivoting on the first largest
-// |B[r][col]|, the pivot row scaled by inv = 1 / pivot, every other row with f != 0
-// reduced by f times the scaled pivot row), on the host: it returns the top-left
-// n x n block of B^-1, column-major.  Plain products and differences (contraction
-// into fused multiply-adds is off), so it agrees bit for bit with the device kernel.
+// The elimination of launch_gj_panel (partial pivoting on the first largest
+// |B[r][col]|) column by column on [B | I] on the host: it returns the top-left n x n
+// block of B^-1, column-major.
 static std::vector<double> coarse_inverse_host(std::vector<double> B, int N, int n) {
 #pragma clang fp contract(off)
   std::vector<double> I((size_t)N * N, 0.);
@@ -123,17 +121,17 @@ static std::vector<double> coarse_inverse_host(std::vector<double> B, int N, int
 }
 
 // Bordered systems up to this many rows are inverted on the host: below it the
-// elimination costs less there than one device launch per column.
+// elimination costs less there than the device launches.
 constexpr int COARSE_HOST_MAX = 96;
 
 // cinv (n x n, column-major, precision T) = the top-left block of B^-1, by
-// Gauss-Jordan with partial pivoting on the device (launch_gj_step; on the host
+// Gauss-Jordan with partial pivoting on the device (launch_gj_panel; on the host
 // for small systems).  The working matrices come from the set-up scratch `tmp`,
 // which a moving body's rebuilds keep from one call to the next.
 template <typename T>
 static void coarse_inverse_device(hipStream_t s, Arena& tmp, const std::vector<double>& B, int n, T* cinv) {
   const int N = (int)std::lround(std::sqrt((double)B.size()));
-  if (N <= COARSE_HOST_MAX) {
+  if (N <= COARSE_HOST_MAX || N > GJ_MAX_ROWS) {
     const std::vector<double> ci = coarse_inverse_host(B, N, n);
     std::vector<T> ct(ci.size());
     for (size_t i = 0; i < ci.size(); i++) ct[i] = T(ci[i]);
@@ -142,15 +140,15 @@ static void coarse_inverse_device(hipStream_t s, Arena& tmp, const std::vector<d
     return;
   }
   const size_t nn = (size_t)N * N;
-  double* m = tmp.alloc<double>(4 * nn + 1);
-  double *b[2] = {m, m + nn}, *id[2] = {m + 2 * nn, m + 3 * nn};
-  int* singular = reinterpret_cast<int*>(m + 4 * nn);
-  h2d(s, b[0], B.data(), nn);
-  launch_gj_identity(s, N, id[0]);
-  HIPCHECK(hipMemsetAsync(singular, 0, sizeof(int), s));
-  for (int col = 0; col < N; col++)
-    launch_gj_step(s, N, col, b[col & 1], id[col & 1], b[(col + 1) & 1], id[(col + 1) & 1], singular);
-  launch_gj_out<T>(s, N, n, id[N & 1], cinv);
+  double* m = tmp.alloc<double>(2 * nn + (size_t)N * GJ_B);
+  double *a[2] = {m, m + nn}, *t = m + 2 * nn;
+  int* p = tmp.alloc<int>(2 * (size_t)N + 1);  // zeroed by the arena
+  int *q = p + N, *singular = p + 2 * N;
+  h2d(s, a[0], B.data(), nn);
+  HIPCHECK(hipMemsetAsync(q, 0xFF, (size_t)N * sizeof(int), s));
+  int z = 0;
+  for (int k = 0; k < N; k += GJ_B, z ^= 1) launch_gj_panel(s, N, k, a[z], a[z ^ 1], t, p, q, singular);
+  launch_gj_out<T>(s, N, n, a[z], p, q, cinv, singular);
   int bad = 0;
   d2h(s, &bad, singular, 1);
   HIPCHECK(hipStreamSynchronize(s));

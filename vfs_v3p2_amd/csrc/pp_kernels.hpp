@@ -73,15 +73,19 @@ void launch_ibface_count(hipStream_t s, Dmda m, Dims d, const double* nv, int im
 void launch_ibface_write(hipStream_t s, Dmda m, Dims d, const double* nv, const double* met9, int immersed,
                          const int* off, IbFace* out);
 
-// Dense inverse of the coarsest level on the device: Gauss-Jordan with partial
-// pivoting on [B | I] (N x N each, row-major), one launch per column col = 0 .. N-1
-// from (bi, ii) to (bo, io) (two buffer pairs in turn); launch_gj_out writes the
-// column-major top-left n x n block of the final I as T.
-void launch_gj_identity(hipStream_t s, int N, double* I);
-void launch_gj_step(hipStream_t s, int N, int col, const double* bi, const double* ii, double* bo, double* io,
-                    int* singular);
+// Dense inverse of the coarsest level on the device: in-place Gauss-Jordan with partial
+// pivoting on an N x N row-major system (N <= GJ_MAX_ROWS), GJ_B columns per call:
+// columns k .. k + GJ_B - 1 from A to B (two buffers in turn).  T holds N * GJ_B
+// doubles; p and q (N ints each, q at -1 before the first call) the pivot rows by column
+// and the columns by pivot row; a singular column sets *singular (0 before).
+// launch_gj_out writes the column-major top-left n x n block of the inverse as T.
+constexpr int GJ_B = 16;
+constexpr int GJ_MAX_ROWS = 2048;
+void launch_gj_panel(hipStream_t s, int N, int k, const double* A, double* B, double* T, int* p, int* q,
+                     int* singular);
 template <typename T>
-void launch_gj_out(hipStream_t s, int N, int n, const double* I, T* cinv);
+void launch_gj_out(hipStream_t s, int N, int n, const double* A, const int* p, const int* q, T* cinv,
+                   const int* singular);
 
 // ---- FP64 operator ----------------------------------------------------------------
 // y = A x on interior vectors; x may be float or double.
