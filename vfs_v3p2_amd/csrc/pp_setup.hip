@@ -14,6 +14,7 @@
 #include <algorithm>
 
 #include "pp_kernels.hpp"
+#include "pp_krylov_dev.hpp"
 #include "pp_stencil.hpp"
 
 namespace pp {
@@ -439,8 +440,26 @@ void launch_ibface_write(hipStream_t s, Dmda m, Dims d, const double* nv, const 
 
 // ---- dense inverse of the coarsest level: in-place Gauss-Jordan in panels of columns
 
-// One panel: columns k .. k + nb - 1 of A (N x N, row-major), one 1024-thread block, R
-// rows per thread with the panel's entries in registers.  Step c picks the pivot, the
+// the largest of the wave's values (all >= 0), for every lane
+__device__ __forceinline__ double wave_max_all(double v) {
+  v = fmax(v, dpp_f64<0x111, 0xF, 0xF>(v));  // row_shr:1
+  v = fmax(v, dpp_f64<0x112, 0xF, 0xF>(v));  // row_shr:2
+  v = fmax(v, dpp_f64<0x114, 0xF, 0xF>(v));  // row_shr:4
+  v = fmax(v, dpp_f64<0x118, 0xF, 0xF>(v));  // row_shr:8
+  v = fmax(v, dpp_f64<0x142, 0xA, 0xF>(v));  // row_bcast:15 into rows 1 and 3
+  v = fmax(v, dpp_f64<0x143, 0xC, 0xF>(v));  // row_bcast:31 into rows 2 and 3
+  union {
+    double d;
+    int i[2];
+  } r;
+  r.d = v;
+  r.i[0] = __builtin_amdgcn_readlane(r.i[0], 63);
+  r.i[1] = __builtin_amdgcn_readlane(r.i[1], 63);
+  return r.d;
+}
+
+// One panel: columns k .. k + nb - 1 of A (N x N, row-major), one block, R rows per
+// thread with the panel's entries in registers.  Step c picks the pivot, the
 // first largest |A[r][k + c]| over the rows that no earlier column took, and eliminates
 // column k + c from every other row of the panel in place: entry (r, k + c) becomes the
 // multiplier of the pivot row.  Rows stay where they are (the column that takes row p is
@@ -448,9 +467,12 @@ void launch_ibface_write(hipStream_t s, Dmda m, Dims d, const double* nv, const 
 // (N x GJ_B) holds the panel, the rows' multipliers of the panel's pivot rows, which
 // k_gj_update applies to the other columns.  A column without a nonzero candidate sets
 // *singular = its number + 1.
-// Bound by the two barriers and the reduction per column, about 1 us each; one launch
-// per column over the whole matrix took 5.8 us per column, this and the update together
-// 1.6 us (a 421-row system 2.45 -> 0.7 ms).
+// Bound by issue on its one CU and by the two barriers per column, so the block has as
+// many waves as the rows need, the pivot row's owner scales it once for everyone and
+// the reduction stays in registers (DPP): 26 us for 16 columns of a 421-row system, 48 us
+// with 1024 threads, shuffles and every thread scaling the pivot row.  One launch per
+// column over the whole matrix took 5.8 us per column; this and the update (9 us per
+// panel) take 2.2 us (2.45 -> 0.95 ms for the inverse).
 template <int R>
 __global__ __launch_bounds__(1024) void k_gj_panel(int N, int k, int nb, const double* __restrict__ A,
                                                    double* __restrict__ T, int* __restrict__ p, int* __restrict__ q,
@@ -458,7 +480,7 @@ __global__ __launch_bounds__(1024) void k_gj_panel(int N, int k, int nb, const d
   __shared__ double best[2][16];
   __shared__ int brow[2][16];
   __shared__ double prow[2][GJ_B];
-  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6;
+  const int t = (int)threadIdx.x, lane = t & 63, w = t >> 6, nw = (int)blockDim.x >> 6;
   if (*singular) return;
   double a[R][GJ_B];
   bool open[R];  // a row of the matrix that no column has taken yet
@@ -483,7 +505,7 @@ __global__ __launch_bounds__(1024) void k_gj_panel(int N, int k, int nb, const d
           row = t + 1024 * u;
         }
       }
-      const double m = wave_max(v);
+      const double m = wave_max_all(v);
       const unsigned long long at = __ballot(v == m);
       const int first = (int)__builtin_ctzll(at);
       const int mrow = __shfl(row, first, 64);
@@ -496,7 +518,7 @@ __global__ __launch_bounds__(1024) void k_gj_panel(int N, int k, int nb, const d
       int br = brow[z][0];
 #pragma unroll
       for (int x = 1; x < 16; x++)
-        if (best[z][x] > bv) {
+        if (x < nw && best[z][x] > bv) {
           bv = best[z][x];
           br = brow[z][x];
         }
@@ -506,30 +528,30 @@ __global__ __launch_bounds__(1024) void k_gj_panel(int N, int k, int nb, const d
         // panels see the flag and write nothing
         br = -1;
         if (t == 0) *singular = k + c + 1;
-        if (t < GJ_B) prow[z][t] = 1.;
+        if (t < GJ_B) prow[z][t] = 0.;
       }
 #pragma unroll
       for (int u = 0; u < R; u++)
         if (t + 1024 * u == br) {
+          // the scaled pivot row, with 1 / pivot in the pivot's place
+          const double inv = 1. / a[u][c];
 #pragma unroll
-          for (int e = 0; e < GJ_B; e++) prow[z][e] = a[u][e];
+          for (int e = 0; e < GJ_B; e++) prow[z][e] = e == c ? inv : a[u][e] * inv;
           p[k + c] = br;
           q[br] = k + c;
+          open[u] = false;
         }
       __syncthreads();
-      const double inv = 1. / prow[z][c];
 #pragma unroll
       for (int u = 0; u < R; u++) {
-        const bool own = t + 1024 * u == br;
-        const double f = own ? -1. : a[u][c];
+        const double f = a[u][c];
+        a[u][c] = 0.;
 #pragma unroll
-        for (int e = 0; e < GJ_B; e++) {
-          if (e == c) continue;
-          const double g = prow[z][e] * inv;
-          a[u][e] = own ? g : a[u][e] - f * g;
+        for (int e = 0; e < GJ_B; e++) a[u][e] -= f * prow[z][e];
+        if (t + 1024 * u == br) {
+#pragma unroll
+          for (int e = 0; e < GJ_B; e++) a[u][e] = prow[z][e];
         }
-        a[u][c] = -f * inv;
-        if (own) open[u] = false;
       }
     }
   }
@@ -562,8 +584,14 @@ __global__ __launch_bounds__(256) void k_gj_update(int N, int k, int nb, const d
     const int c = e / 32, j = j0 + e % 32;
     pv[c][e % 32] = (c < nb && j < N) ? A[(size_t)p[k + c] * N + j] : 0.;
   }
-  __syncthreads();
   const int jl = t & 31, j = j0 + jl;
+  double base[8];  // in flight with the tiles
+#pragma unroll
+  for (int x = 0; x < 8; x++) {
+    const int r = r0 + (t >> 5) + 8 * x;
+    base[x] = (r < N && j < N) ? A[(size_t)r * N + j] : 0.;
+  }
+  __syncthreads();
   if (j >= N) return;
 #pragma unroll
   for (int x = 0; x < 8; x++) {
@@ -576,7 +604,7 @@ __global__ __launch_bounds__(256) void k_gj_update(int N, int k, int nb, const d
       bool piv = false;
 #pragma unroll
       for (int c = 0; c < GJ_B; c++) piv = piv || pr[c] == r;
-      v = piv ? 0. : A[(size_t)r * N + j];
+      v = piv ? 0. : base[x];
 #pragma unroll
       for (int c = 0; c < GJ_B; c++) v += tp[rl][c] * pv[c][jl];
     }
@@ -600,7 +628,7 @@ void launch_gj_panel(hipStream_t s, int N, int k, const double* A, double* B, do
                      int* singular) {
   if (N > GJ_MAX_ROWS) throw StatusError(1, "dense inverse: system too large");
   const int nb = std::min(GJ_B, N - k);
-  if (N <= 1024) k_gj_panel<1><<<1, 1024, 0, s>>>(N, k, nb, A, T, p, q, singular);
+  if (N <= 1024) k_gj_panel<1><<<1, (N + 63) / 64 * 64, 0, s>>>(N, k, nb, A, T, p, q, singular);
   else k_gj_panel<2><<<1, 1024, 0, s>>>(N, k, nb, A, T, p, q, singular);
   HIPCHECK(hipGetLastError());
   k_gj_update<<<dim3((N + 31) / 32, (N + 63) / 64), 256, 0, s>>>(N, k, nb, A, T, p, B, singular);
