@@ -719,20 +719,34 @@ void launch_ucont_ghosts(hipStream_t s, Dmda m, double* ucont) {
   HIPCHECK(hipGetLastError());
 }
 
-void launch_c2c(hipStream_t s, Dmda m, Dims d, const double* met9, const uint8_t* cls, const double* nvert,
-                const double* ucont, double* ucat, double* scratch, const int bc[6]) {
-  k_c2c_core<<<cell_grid(d), kBlk, 0, s>>>(m, d, met9, cls, ucont, ucat);
-  HIPCHECK(hipGetLastError());
+// the boundary points of Contra2Cart: periodic copies with a snapshot, the boundary rules
+static void c2c_bounds(hipStream_t s, Dmda m, const double* nvert, double* ucat, double* scratch, const int bc[6]) {
   k_vec_ghosts<<<bnd_blocks(m), 256, 0, s>>>(m, ucat, scratch);
   HIPCHECK(hipGetLastError());
   k_c2c_bc<<<bnd_blocks(m), 256, 0, s>>>(m, nvert, scratch, ucat, bc[0], bc[1], bc[2], bc[3], bc[4], bc[5]);
   HIPCHECK(hipGetLastError());
-  k_c2c_solid<<<cell_grid(d), kBlk, 0, s>>>(d, m, cls, ucat);
-  HIPCHECK(hipGetLastError());
+}
+
+static void c2c_periodic(hipStream_t s, Dmda m, double* ucat) {
   if (m.per[0] || m.per[1] || m.per[2]) {
     k_vec_ghosts<<<bnd_blocks(m), 256, 0, s>>>(m, ucat, nullptr);
     HIPCHECK(hipGetLastError());
   }
+}
+
+void launch_c2c(hipStream_t s, Dmda m, Dims d, const double* met9, const uint8_t* cls, const double* nvert,
+                const double* ucont, double* ucat, double* scratch, const int bc[6]) {
+  k_c2c_core<<<cell_grid(d), kBlk, 0, s>>>(m, d, met9, cls, ucont, ucat);
+  HIPCHECK(hipGetLastError());
+  c2c_bounds(s, m, nvert, ucat, scratch, bc);
+  k_c2c_solid<<<cell_grid(d), kBlk, 0, s>>>(d, m, cls, ucat);
+  HIPCHECK(hipGetLastError());
+  c2c_periodic(s, m, ucat);
+}
+
+void launch_c2c_again(hipStream_t s, Dmda m, const double* nvert, double* ucat, double* scratch, const int bc[6]) {
+  c2c_bounds(s, m, nvert, ucat, scratch, bc);
+  c2c_periodic(s, m, ucat);
 }
 
 void launch_divest(hipStream_t s, Dims d, const uint32_t* code, const double* aj, const double* r, double* partial,

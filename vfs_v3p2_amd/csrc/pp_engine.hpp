@@ -382,8 +382,19 @@ struct vfs_pp_handle {
   pp::Arena ar;   // buffers sized by the grid alone
   pp::Arena geo;  // buffers of the current geometry (hierarchy, face list), renewed by each set-up
   pp::Arena setup_tmp;  // set-up scratch, kept between set-ups of a moving body
-  // device bytes the handle holds: grid-sized buffers, the geometry's and set-up scratch
-  size_t resident_bytes() const { return ar.total() + geo.total() + setup_tmp.total(); }
+  // device bytes the handle holds: grid-sized buffers, the geometry's, set-up scratch and
+  // momentum work vectors
+  size_t resident_bytes() const { return ar.total() + geo.total() + setup_tmp.total() + mom.total(); }
+  pp::Arena mom;  // momentum work vectors, from the first momentum step on (mom_buf)
+  std::vector<std::pair<double*, size_t>> mom_bufs;
+  // work vector q of the momentum steps, at least n doubles; kept by the handle, since
+  // allocating and freeing about 1 GB per call cost an implicit step of 1.2 M cells about 2 ms.  Only
+  // points the steps write are ever read, and a handle's grid never changes.
+  double* mom_buf(size_t q, size_t n) {
+    if (mom_bufs.size() <= q) mom_bufs.resize(q + 1, {nullptr, 0});
+    if (mom_bufs[q].second < n) mom_bufs[q] = {mom.alloc<double>(n), n};
+    return mom_bufs[q].first;
+  }
   double* hstage = nullptr;   // device copies of vfs_pp_project's host arrays (8 M doubles, from ar)
   int batch_refs = 0;         // batches / server slots the handle is bound to (0 or 1)
   int immersed_ref = 0;       // the caller's `immersed` as given (grid.immersed holds the VolumeFlux variant)
@@ -435,6 +446,7 @@ constexpr int RED_DIV = 330;   // max |aj div u|
 constexpr int RED_DIVEST = 340;  // max |aj r| at the last true-residual check
 constexpr int RED_SETUP = 350;   // set-up statistics: 4 values
 constexpr int RED_LAMBDA = 1024;  // set-up power iterations: 12 norms per level (hpin only)
+constexpr int RED_MOM = 2048;     // momentum steps' dot products: 128 values (hpin only)
 constexpr int RED_NUINV2 = 400;  // 1 / |U_l|^2 of the lazily normalised basis (up to 64)
 
 // engine functions shared with the batched engine (pp_engine.hip)

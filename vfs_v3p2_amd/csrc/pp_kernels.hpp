@@ -124,6 +124,10 @@ void launch_projection(hipStream_t s, Dmda m, Dims d, const double* g, const uin
 void launch_ucont_ghosts(hipStream_t s, Dmda m, double* ucont);
 void launch_c2c(hipStream_t s, Dmda m, Dims d, const double* met9, const uint8_t* cls, const double* nvert,
                 const double* ucont, double* ucat, double* scratch, const int bctype[6]);
+// a second launch_c2c on the same Ucont and the first one's Ucat: the interior would come
+// out as it is, so only the boundary points are taken again (an edge between two walls
+// reads the first pass's values)
+void launch_c2c_again(hipStream_t s, Dmda m, const double* nvert, double* ucat, double* scratch, const int bctype[6]);
 void launch_divest(hipStream_t s, Dims d, const uint32_t* code, const double* aj, const double* r, double* partial,
                    int* nblk);
 void launch_divergence(hipStream_t s, Dmda m, Dims d, const uint32_t* code, const double* aj, const double* ucont,

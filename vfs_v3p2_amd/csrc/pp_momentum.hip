@@ -10,7 +10,7 @@
 // whose Ucat carries their results in IB-adjacent cells (Contra2Cart leaves
 // those cells as they are).
 //
-// One thread per DMDA point in every kernel.  The face fluxes of the three
+// One thread per DMDA point in every kernel over the box.  The face fluxes of the three
 // families are written to DMDA arrays (convective and viscous apart, since the
 // cell step takes a fourth-order difference of the convective ones), their
 // periodic ghosts copied, then the cell divergence Fp and the contravariant
@@ -19,6 +19,7 @@
 #include <limits>
 
 #include "pp_engine.hpp"
+#include "pp_path_dev.hpp"
 
 namespace pp {
 
@@ -39,11 +40,16 @@ struct V3 {
   double x[3];
 };
 
+// this thread's DMDA point: 256 consecutive points per block (a row of mx points never
+// fills whole 64-lane tiles), blocks in XCD order (points adjacent in k share an L2)
 __device__ __forceinline__ bool dmda_point(const Dmda& m, int& i, int& j, int& k) {
-  i = blockIdx.x * 64 + threadIdx.x;
-  j = blockIdx.y * 4 + threadIdx.y;
-  k = blockIdx.z;
-  return i < m.mx && j < m.my;
+  const uint32_t e = xcd_block().x * 256u + threadIdx.x, mx = (uint32_t)m.mx, pl = mx * (uint32_t)m.my;
+  if (e >= pl * (uint32_t)m.mz) return false;
+  k = (int)(e / pl);
+  const uint32_t r = e - (uint32_t)k * pl;
+  j = (int)(r / mx);
+  i = (int)(r - (uint32_t)j * mx);
+  return true;
 }
 
 // the periodic image of a ghost point (the `if(periodic)` copies,
@@ -74,30 +80,58 @@ __global__ __launch_bounds__(256) void k_mm_local_ucont(Dmda m, const double* __
   lu[3 * p + 2] = u[3 * s + 2];
 }
 
-// Compute_du_i / _j / _k (inline.h:406-611): du[c][e] = d U_c / d xi_e at face D
+// Ucat at the ten points Compute_du_i / _j / _k may read for face D of point p: the two
+// cells of the face, and for each cross axis the four cells beside them.  All of them
+// and the masks are loaded before any case is decided (every one is a point of the
+// array), so the face waits for memory once instead of once per branch.  The kernels
+// stream about 184 B per point and family; with that, flat 256-point blocks and the XCD
+// order a family takes 112 us at 192x96x128 (155 before; 4.1 TB/s).
+struct FaceIn {
+  double u[10][3];  // p, p + sd; then per cross axis: +e of p and p + sd, -e of p and p + sd
+  double nv[8];     // per cross axis: +e of p, p + sd, -e of p, p + sd
+};
 template <int D>
-__device__ __forceinline__ void face_du(const size_t (&st)[3], size_t p, const double* __restrict__ u,
-                                        const double* __restrict__ nv, double (&du)[3][3]) {
+__device__ __forceinline__ void face_load(const size_t (&st)[3], size_t p, const double* __restrict__ u,
+                                          const double* __restrict__ nv, FaceIn& f) {
+  constexpr int E[2] = {D == 0 ? 1 : 0, D == 2 ? 1 : 2};
   const size_t sd = st[D];
 #pragma unroll
-  for (int c = 0; c < 3; c++) du[c][D] = u[3 * (p + sd) + c] - u[3 * p + c];
+  for (int x = 0; x < 2; x++) {
+    const size_t se = st[E[x]];
+    const size_t q[4] = {p + se, p + sd + se, p - se, p + sd - se};
 #pragma unroll
-  for (int e = 0; e < 3; e++) {
-    if (e == D) continue;
-    const size_t se = st[e];
-    if (nv[p + se] > 0.1 || nv[p + sd + se] > 0.1) {
+    for (int y = 0; y < 4; y++) {
+      f.nv[4 * x + y] = nv[q[y]];
 #pragma unroll
-      for (int c = 0; c < 3; c++)
-        du[c][e] = (u[3 * (p + sd) + c] + u[3 * p + c] - u[3 * (p + sd - se) + c] - u[3 * (p - se) + c]) * 0.5;
-    } else if (nv[p - se] > 0.1 || nv[p + sd - se] > 0.1) {
+      for (int c = 0; c < 3; c++) f.u[2 + 4 * x + y][c] = u[3 * q[y] + c];
+    }
+  }
 #pragma unroll
-      for (int c = 0; c < 3; c++)
-        du[c][e] = (u[3 * (p + sd + se) + c] + u[3 * (p + se) + c] - u[3 * (p + sd) + c] - u[3 * p + c]) * 0.5;
-    } else {
+  for (int c = 0; c < 3; c++) {
+    f.u[0][c] = u[3 * p + c];
+    f.u[1][c] = u[3 * (p + sd) + c];
+  }
+}
+
+// Compute_du_i / _j / _k (inline.h:406-611): du[c][e] = d U_c / d xi_e at face D
+template <int D>
+__device__ __forceinline__ void face_du(const FaceIn& f, double (&du)[3][3]) {
+  constexpr int E[2] = {D == 0 ? 1 : 0, D == 2 ? 1 : 2};
 #pragma unroll
-      for (int c = 0; c < 3; c++)
-        du[c][e] =
-            (u[3 * (p + sd + se) + c] + u[3 * (p + se) + c] - u[3 * (p + sd - se) + c] - u[3 * (p - se) + c]) * 0.25;
+  for (int c = 0; c < 3; c++) du[c][D] = f.u[1][c] - f.u[0][c];
+#pragma unroll
+  for (int x = 0; x < 2; x++) {
+    const int e = E[x];
+    const double(&ph)[3] = f.u[2 + 4 * x], (&qh)[3] = f.u[3 + 4 * x];  // +e of p and of p + sd
+    const double(&pl)[3] = f.u[4 + 4 * x], (&ql)[3] = f.u[5 + 4 * x];  // -e
+    const bool hi = f.nv[4 * x] > 0.1 || f.nv[4 * x + 1] > 0.1, lo = f.nv[4 * x + 2] > 0.1 || f.nv[4 * x + 3] > 0.1;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      // upper pair: the cells themselves when an upper cell is IB; lower pair: the cells
+      // when only a lower one is
+      const double q1 = hi ? f.u[1][c] : qh[c], p1 = hi ? f.u[0][c] : ph[c];
+      const double q0 = !hi && lo ? f.u[1][c] : ql[c], p0 = !hi && lo ? f.u[0][c] : pl[c];
+      du[c][e] = (q1 + p1 - q0 - p0) * (hi || lo ? 0.5 : 0.25);
     }
   }
 }
@@ -116,14 +150,17 @@ __global__ __launch_bounds__(256) void k_mm_faces(Dmda m, MomIn in, const double
   const size_t st[3] = {1, (size_t)m.mx, (size_t)m.mx * m.my};
   const size_t p = m.idx(i, j, k), sd = st[D];
   const double* __restrict__ nv = in.nv;
+  FaceIn fi;
+  face_load<D>(st, p, ucat, nv, fi);
   const double ajc = in.faj[D][p];
+  const double nv0 = nv[p], nvd = nv[p + sd], fl = uc[3 * p + D];
   double mt[3][3];
 #pragma unroll
   for (int e = 0; e < 3; e++)
 #pragma unroll
     for (int x = 0; x < 3; x++) mt[e][x] = in.fm[D][e][3 * p + x];
   double du[3][3];
-  face_du<D>(st, p, ucat, nv, du);
+  face_du<D>(fi, du);
   double g[3];
 #pragma unroll
   for (int e = 0; e < 3; e++) g[e] = mt[e][0] * mt[D][0] + mt[e][1] * mt[D][1] + mt[e][2] * mt[D][2];
@@ -133,6 +170,7 @@ __global__ __launch_bounds__(256) void k_mm_faces(Dmda m, MomIn in, const double
 #pragma unroll
     for (int x = 0; x < 3; x++) r[c][x] = du[c][0] * mt[0][x] + du[c][1] * mt[1][x] + du[c][2] * mt[2][x];
   const int pd = pos[D], md = mm[D];
+  // the outer points of the fourth-order face value, the face's own cells at its ends
   size_t L = p - sd, R = p + 2 * sd;
   if (pd == 0 || pd == md - 2) {
     if (m.per[D]) {
@@ -142,23 +180,35 @@ __global__ __launch_bounds__(256) void k_mm_faces(Dmda m, MomIn in, const double
       L = p;
       R = p + sd;
     }
-  } else if (nv[L] + nv[R] > 0.1) {
-    L = p;
-    R = p + sd;
   }
-  double ucon = uc[3 * p + D];
+  const bool ends = pd == 0 || pd == md - 2;
+  const double nl = nv[L], nr = nv[R];
+  double ul[3], ur[3];
+#pragma unroll
+  for (int c = 0; c < 3; c++) {
+    ul[c] = ucat[3 * L + c];
+    ur[c] = ucat[3 * R + c];
+  }
+  double ucon = fl;
   if (m.per[D] && (pd == 0 || pd == md - 2)) ucon = uc[3 * (size_t)((long long)p + (long long)(md - 2 - pd) * (long long)sd) + D];
-  if (D == 2 && k == m.mz - 2 && in.bc5 == 4 && (int)nv[p] == 0) ucon = uc[3 * (p - sd) + 2];
+  if (D == 2 && k == m.mz - 2 && in.bc5 == 4 && (int)nv0 == 0) ucon = uc[3 * (p - sd) + 2];
+  if (!ends && nl + nr > 0.1) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      ul[c] = fi.u[0][c];
+      ur[c] = fi.u[1][c];
+    }
+  }
   const double up = -0.5 * (ucon + fabs(ucon));
   const double um = -0.5 * (ucon - fabs(ucon));
   double dv[3];
-  if (in.immersed && pd != md - 2 && nv[p] > 0.1) {
+  if (in.immersed && pd != md - 2 && nv0 > 0.1) {
 #pragma unroll
     for (int c = 0; c < 3; c++)
       dv[c] = um * (0.125 * (-ucat[3 * (p + 2 * sd) + c] - 2. * ucat[3 * (p + sd) + c] + 3. * ucat[3 * p + c]) +
                     ucat[3 * (p + sd) + c]) +
               up * (0.125 * (-ucat[3 * p + c] - 2. * ucat[3 * p + c] + 3. * ucat[3 * (p + sd) + c]) + ucat[3 * p + c]);
-  } else if (in.immersed && pd != 0 && nv[p + sd] > 0.1) {
+  } else if (in.immersed && pd != 0 && nvd > 0.1) {
 #pragma unroll
     for (int c = 0; c < 3; c++)
       dv[c] = um * (0.125 * (-ucat[3 * (p + sd) + c] - 2. * ucat[3 * (p + sd) + c] + 3. * ucat[3 * p + c]) +
@@ -166,12 +216,10 @@ __global__ __launch_bounds__(256) void k_mm_faces(Dmda m, MomIn in, const double
               up * (0.125 * (-ucat[3 * (p - sd) + c] - 2. * ucat[3 * p + c] + 3. * ucat[3 * (p + sd) + c]) +
                     ucat[3 * p + c]);
   } else {
-    const double fl = uc[3 * p + D];
 #pragma unroll
-    for (int c = 0; c < 3; c++)
-      dv[c] = -fl * 0.0625 * (-ucat[3 * L + c] + 9. * ucat[3 * p + c] + 9. * ucat[3 * (p + sd) + c] - ucat[3 * R + c]);
+    for (int c = 0; c < 3; c++) dv[c] = -fl * 0.0625 * (-ul[c] + 9. * fi.u[0][c] + 9. * fi.u[1][c] - ur[c]);
   }
-  if (nv[p] + nv[p + sd] > 0.1 && in.immersed == 3) dv[0] = dv[1] = dv[2] = 0.;
+  if (nv0 + nvd > 0.1 && in.immersed == 3) dv[0] = dv[1] = dv[2] = 0.;
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     div[3 * p + c] = dv[c];
@@ -183,16 +231,20 @@ __global__ __launch_bounds__(256) void k_mm_faces(Dmda m, MomIn in, const double
   }
 }
 
-// whole-vector periodic ghost copies of n3 DMDA vector arrays, in place
+// whole-vector periodic ghost copies of narr DMDA vector arrays, in place; one thread per
+// boundary point of the box (a pass over the whole box took 39 us at 192x96x128, this
+// one 14 us, the mean of its six- and one-array launches)
 __global__ __launch_bounds__(256) void k_mm_periodic(Dmda m, double* a0, double* a1, double* a2, double* a3,
                                                      double* a4, double* a5, int narr) {
   int i, j, k;
-  if (!dmda_point(m, i, j, k)) return;
+  if (!boundary_point(m, blockIdx.x * 256u + threadIdx.x, i, j, k)) return;
   size_t s;
   if (!ghost_image(m, i, j, k, s)) return;
   const size_t p = m.idx(i, j, k);
   double* arr[6] = {a0, a1, a2, a3, a4, a5};
-  for (int q = 0; q < narr; q++) {
+#pragma unroll
+  for (int q = 0; q < 6; q++) {
+    if (q >= narr) break;
     double* a = arr[q];
     a[3 * p] = a[3 * s];
     a[3 * p + 1] = a[3 * s + 1];
@@ -258,12 +310,55 @@ __global__ __launch_bounds__(256) void k_mm_fp(Dmda m, const double* __restrict_
   }
 }
 
-// the contravariant right-hand side (momentum.c:1750-1965) at every DMDA point;
-// acc = 0: Rhs starts at zero (the caller's VecSet), acc = 1: the terms add to what
-// Rhs holds (FormFunction_SNES adds them to its time terms); boundary-plane points
-// end at zero either way
+struct Bc6 {
+  int b[6];
+};
+
+// The components of point (i, j, k) that FormFunction_SNES zeroes (momentum.c:2323-2356):
+// bctype 1 / -1 walls zero the normal flux on their wall face (i = 0 and i = mx - 2
+// for the two i walls, likewise j and k), cavity (2) and couette (12) walls the j
+// faces, slip (10) walls the i or j faces away from the boundary rows of the other
+// axes (the rules written at i = mx - 1 land on i = mx - 2).
+__device__ __forceinline__ void wall_zero(const Dmda& m, const Bc6& bc, int i, int j, int k, double (&u)[3]) {
+  const int* b = bc.b;
+  const bool ik = j != 0 && j != m.my - 1 && k != 0 && k != m.mz - 1;
+  const bool jk = i != 0 && i != m.mx - 1 && k != 0 && k != m.mz - 1;
+  const bool zx = (i == 0 && (b[0] == 1 || b[0] == -1)) || (i == m.mx - 2 && (b[1] == 1 || b[1] == -1)) ||
+                  (b[0] == 10 && i == 0 && ik) || (b[1] == 10 && i == m.mx - 2 && ik);
+  const bool zy = (j == 0 && (b[2] == 1 || b[2] == -1 || b[2] == 12)) ||
+                  (j == m.my - 2 && (b[3] == 1 || b[3] == -1 || b[3] == 2 || b[3] == 12)) ||
+                  (b[2] == 10 && j == 0 && jk) || ((b[3] == 10 || b[3] == -10) && j == m.my - 2 && jk);
+  const bool zz = (k == 0 && (b[4] == 1 || b[4] == -1)) || (k == m.mz - 2 && (b[5] == 1 || b[5] == -1));
+  if (zx) u[0] = 0.;
+  if (zy) u[1] = 0.;
+  if (zz) u[2] = 0.;
+}
+
+// What FormFunction_SNES puts around the right-hand side: before it the time terms of
+// U with its wall components zeroed, summed as the VecAXPY sequence from a zero vector
+// does, -(Uz - Uo)/dt (bdf1) or -(1.5 Uz - 2 Uo + 0.5 Urm1)/dt; after it 0.5 RHS_o (bdf1,
+// when given) and -dP.
+// U is u, or u + h v (v given).  With f0 the kernel stores (F - f0) / h, the directional
+// difference of a Jacobian-free product, instead of F.
+struct SnesTerms {
+  Bc6 bc;
+  const double *u, *v, *uo, *urm1, *rhs_o, *dp, *f0;
+  int bdf1;
+  double dt, h;
+};
+// component c of U at array position q
+__device__ __forceinline__ double snes_u(const double* __restrict__ u, const double* __restrict__ v, double h,
+                                         size_t q) {
+  return v ? u[q] + h * v[q] : u[q];
+}
+
+// the contravariant right-hand side (momentum.c:1750-1965) at every DMDA point.
+// SNES: its terms add to FormFunction_SNES's time terms and are followed by its tail
+// (boundary-plane points start at zero either way), so F is written once instead of three
+// times and read not at all; else Rhs starts at zero (the caller's VecSet).
+template <bool SNES>
 __global__ __launch_bounds__(256) void k_mm_rhs(Dmda m, MomIn in, const double* __restrict__ fp, double scale,
-                                                int acc, double* __restrict__ rhs) {
+                                                SnesTerms t, double* __restrict__ rhs) {
   int i, j, k;
   if (!dmda_point(m, i, j, k)) return;
   const size_t st[3] = {1, (size_t)m.mx, (size_t)m.mx * m.my};
@@ -271,12 +366,24 @@ __global__ __launch_bounds__(256) void k_mm_rhs(Dmda m, MomIn in, const double* 
   const int pos[3] = {i, j, k}, mq[3] = {m.mx, m.my, m.mz};
   double out[3] = {0., 0., 0.};
   const bool interior = i > 0 && j > 0 && k > 0 && i < m.mx - 1 && j < m.my - 1 && k < m.mz - 1;
-  if (interior && acc) {
-    out[0] = rhs[3 * p];
-    out[1] = rhs[3 * p + 1];
-    out[2] = rhs[3 * p + 2];
-  }
   if (interior) {
+    if constexpr (SNES) {
+      double uz[3] = {snes_u(t.u, t.v, t.h, 3 * p), snes_u(t.u, t.v, t.h, 3 * p + 1), snes_u(t.u, t.v, t.h, 3 * p + 2)};
+      wall_zero(m, t.bc, i, j, k, uz);
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        double r = 0.;
+        if (t.bdf1) {
+          r = r + -1. / t.dt * uz[c];
+          r = r + 1. / t.dt * t.uo[3 * p + c];
+        } else {
+          r = r + -1.5 / t.dt * uz[c];
+          r = r + 2. / t.dt * t.uo[3 * p + c];
+          r = r + -0.5 / t.dt * t.urm1[3 * p + c];
+        }
+        out[c] = r;
+      }
+    }
     const double* nv = in.nv;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
@@ -289,10 +396,15 @@ __global__ __launch_bounds__(256) void k_mm_rhs(Dmda m, MomIn in, const double* 
                 in.faj[d][p];
       if (nv[p] + nv[p + st[d]] > 0.1 || (!m.per[d] && pos[d] == mq[d] - 2)) out[d] = 0.;
     }
-  } else {
+  }
+  if constexpr (SNES) {
 #pragma unroll
-    for (int a = 0; a < 3; a++)
-      if (pos[a] == mq[a] - 2 && !m.per[a]) out[a] = 0.;
+    for (int c = 0; c < 3; c++) {
+      double r = out[c];
+      if (t.rhs_o) r = r + 0.5 * t.rhs_o[3 * p + c];
+      r = r + -1. * t.dp[3 * p + c];
+      out[c] = t.f0 ? (r - t.f0[3 * p + c]) / t.h : r;
+    }
   }
   rhs[3 * p] = out[0];
   rhs[3 * p + 1] = out[1];
@@ -315,33 +427,29 @@ __global__ __launch_bounds__(256) void k_mm_copy(size_t n, const double* __restr
 }
 
 // ------------------------------------------------------------ implicit form
-struct Bc6 {
-  int b[6];
-};
-
-// U with the wall components FormFunction_SNES zeroes (momentum.c:2323-2356):
-// bctype 1 / -1 walls zero the normal flux on their wall face (i = 0 and i = mx - 2
-// for the two i walls, likewise j and k), cavity (2) and couette (12) walls the j
-// faces, slip (10) walls the i or j faces away from the boundary rows of the other
-// axes.  Each point zeroes its own components (the rules written at i = mx - 1
-// land on i = mx - 2).
-__global__ __launch_bounds__(256) void k_mm_bc_zero(Dmda m, Bc6 bc, const double* __restrict__ u,
-                                                    double* __restrict__ uz) {
+// U (u, or u + h v) with its wall components zeroed (uz, when given) and its local copy
+// with the whole-vector periodic ghosts of that (lu)
+__global__ __launch_bounds__(256) void k_mm_local_zeroed(Dmda m, Bc6 bc, const double* __restrict__ u,
+                                                         const double* __restrict__ v, double h,
+                                                         double* __restrict__ uz, double* __restrict__ lu) {
   int i, j, k;
   if (!dmda_point(m, i, j, k)) return;
   const size_t p = m.idx(i, j, k);
-  const int* b = bc.b;
-  const bool ik = j != 0 && j != m.my - 1 && k != 0 && k != m.mz - 1;
-  const bool jk = i != 0 && i != m.mx - 1 && k != 0 && k != m.mz - 1;
-  const bool zx = (i == 0 && (b[0] == 1 || b[0] == -1)) || (i == m.mx - 2 && (b[1] == 1 || b[1] == -1)) ||
-                  (b[0] == 10 && i == 0 && ik) || (b[1] == 10 && i == m.mx - 2 && ik);
-  const bool zy = (j == 0 && (b[2] == 1 || b[2] == -1 || b[2] == 12)) ||
-                  (j == m.my - 2 && (b[3] == 1 || b[3] == -1 || b[3] == 2 || b[3] == 12)) ||
-                  (b[2] == 10 && j == 0 && jk) || ((b[3] == 10 || b[3] == -10) && j == m.my - 2 && jk);
-  const bool zz = (k == 0 && (b[4] == 1 || b[4] == -1)) || (k == m.mz - 2 && (b[5] == 1 || b[5] == -1));
-  uz[3 * p] = zx ? 0. : u[3 * p];
-  uz[3 * p + 1] = zy ? 0. : u[3 * p + 1];
-  uz[3 * p + 2] = zz ? 0. : u[3 * p + 2];
+  size_t s;
+  if (!ghost_image(m, i, j, k, s)) s = p;
+  const int sk = (int)(s / ((size_t)m.mx * m.my)), sj = (int)(s / m.mx) % m.my, si = (int)(s % m.mx);
+  double x[3] = {snes_u(u, v, h, 3 * s), snes_u(u, v, h, 3 * s + 1), snes_u(u, v, h, 3 * s + 2)};
+  wall_zero(m, bc, si, sj, sk, x);
+  lu[3 * p] = x[0];
+  lu[3 * p + 1] = x[1];
+  lu[3 * p + 2] = x[2];
+  if (uz) {
+    double w[3] = {snes_u(u, v, h, 3 * p), snes_u(u, v, h, 3 * p + 1), snes_u(u, v, h, 3 * p + 2)};
+    wall_zero(m, bc, i, j, k, w);
+    uz[3 * p] = w[0];
+    uz[3 * p + 1] = w[1];
+    uz[3 * p + 2] = w[2];
+  }
 }
 
 // IB_BC (momentum.c:2037-2220) on the Ucont that Formfunction_2 reads, for a body
@@ -367,42 +475,6 @@ __global__ __launch_bounds__(256) void k_mm_ib_bc(Dmda m, Bc6 bc, int immersed, 
   ul[3 * p] = zx ? 0. : u[3 * p];
   ul[3 * p + 1] = zy ? 0. : u[3 * p + 1];
   ul[3 * p + 2] = zz ? 0. : u[3 * p + 2];
-}
-
-// the time terms, summed as the VecAXPY sequence from a zero vector does:
-// -(Uz - Uo)/dt (coeff 1) or -(1.5 Uz - 2 Uo + 0.5 Urm1)/dt
-__global__ __launch_bounds__(256) void k_mm_time(size_t n3, const double* __restrict__ uz,
-                                                 const double* __restrict__ uo, const double* __restrict__ urm1,
-                                                 int bdf1, double dt, double* __restrict__ f) {
-  const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (q >= n3) return;
-  double r = 0.;
-  if (bdf1) {
-    r = r + -1. / dt * uz[q];
-    r = r + 1. / dt * uo[q];
-  } else {
-    r = r + -1.5 / dt * uz[q];
-    r = r + 2. / dt * uo[q];
-    r = r + -0.5 / dt * urm1[q];
-  }
-  f[q] = r;
-}
-
-// F += 0.5 RHS_o (coeff 1), F += -1 dP
-__global__ __launch_bounds__(256) void k_mm_tail(size_t n3, const double* __restrict__ rhs_o,
-                                                 const double* __restrict__ dp, double* __restrict__ f) {
-  const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (q >= n3) return;
-  double r = f[q];
-  if (rhs_o) r = r + 0.5 * rhs_o[q];
-  f[q] = r + -1. * dp[q];
-}
-
-// w = (a - b) / h
-__global__ __launch_bounds__(256) void k_mm_fd(size_t n3, const double* __restrict__ a, const double* __restrict__ b,
-                                               double h, double* __restrict__ w) {
-  const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (q < n3) w[q] = (a[q] - b[q]) / h;
 }
 
 // y = x + a v
@@ -433,28 +505,32 @@ __global__ __launch_bounds__(256) void k_mm_bc_post(Dmda m, Bc6 bc, double* __re
   if ((wall(b[4]) && k == 0) || (wall(b[5]) && k == m.mz - 2)) u[3 * p + 2] = 0.;
 }
 
-dim3 box_grid(const Dmda& m) { return dim3((m.mx + 63) / 64, (m.my + 3) / 4, m.mz); }
+unsigned box_grid(const Dmda& m) { return (unsigned)((m.n() + 255) / 256); }
 
-// Formfunction_2 on device arrays; ws holds 7 DMDA vector arrays (3 M doubles each)
+// Formfunction_2 on device arrays; ws holds 8 DMDA vector arrays (3 M doubles each), the
+// first of them the local Ucont, which a caller that has it there passes as ucont null.
+// snes: the terms FormFunction_SNES adds around it.
 void formfunction2(hipStream_t s, const Dmda& m, const MomIn& in, const double* ucont, const double* ucat,
-                   double ren, double scale, double* ws, double* rhs, bool acc = false) {
+                   double ren, double scale, double* ws, double* rhs, const SnesTerms* snes = nullptr) {
   const size_t M3 = 3 * m.n();
   double* lu = ws;
   double* dv[3] = {ws + M3, ws + 2 * M3, ws + 3 * M3};
   double* vs[3] = {ws + 4 * M3, ws + 5 * M3, ws + 6 * M3};
   double* fp = ws + 7 * M3;
-  const dim3 gr = box_grid(m), bl(64, 4);
+  const unsigned gr = box_grid(m), bl = 256;
+  const unsigned bnd = (boundary_count(m) + 255) / 256;
   const double nu = 1. / ren;
-  k_mm_local_ucont<<<gr, bl, 0, s>>>(m, ucont, lu);
+  if (ucont) k_mm_local_ucont<<<gr, bl, 0, s>>>(m, ucont, lu);
   k_mm_faces<0><<<gr, bl, 0, s>>>(m, in, lu, ucat, nu, dv[0], vs[0]);
   k_mm_faces<1><<<gr, bl, 0, s>>>(m, in, lu, ucat, nu, dv[1], vs[1]);
   k_mm_faces<2><<<gr, bl, 0, s>>>(m, in, lu, ucat, nu, dv[2], vs[2]);
   if (m.per[0] || m.per[1] || m.per[2])
-    k_mm_periodic<<<gr, bl, 0, s>>>(m, dv[0], dv[1], dv[2], vs[0], vs[1], vs[2], 6);
+    k_mm_periodic<<<bnd, 256, 0, s>>>(m, dv[0], dv[1], dv[2], vs[0], vs[1], vs[2], 6);
   k_mm_fp<<<gr, bl, 0, s>>>(m, in.nv, dv[0], dv[1], dv[2], vs[0], vs[1], vs[2], fp);
   if (m.per[0] || m.per[1] || m.per[2])
-    k_mm_periodic<<<gr, bl, 0, s>>>(m, fp, nullptr, nullptr, nullptr, nullptr, nullptr, 1);
-  k_mm_rhs<<<gr, bl, 0, s>>>(m, in, fp, scale, acc ? 1 : 0, rhs);
+    k_mm_periodic<<<bnd, 256, 0, s>>>(m, fp, nullptr, nullptr, nullptr, nullptr, nullptr, 1);
+  if (snes) k_mm_rhs<true><<<gr, bl, 0, s>>>(m, in, fp, scale, *snes, rhs);
+  else k_mm_rhs<false><<<gr, bl, 0, s>>>(m, in, fp, scale, SnesTerms{}, rhs);
   HIPCHECK(hipGetLastError());
 }
 
@@ -483,12 +559,11 @@ struct ImplicitMomentum {
   Dmda m;
   Dims d;
   MomIn in;
-  const vfs_pp_handle* h;
+  vfs_pp_handle* h;
   Bc6 bc;
   const double *dp, *uo, *urm1, *rhs_o;
   double ren, dt, coeff;
   size_t n3;
-  Arena ar;
   double *ws = nullptr, *uz = nullptr, *ul = nullptr, *partial = nullptr, *red = nullptr;
   bool ib_bc = false;  // IB_BC changes the Ucont Formfunction_2 reads (immersed 3 or slip faces)
   double* hpin = nullptr;  // pinned host mirror of red
@@ -499,37 +574,34 @@ struct ImplicitMomentum {
 
   void init() {
     n3 = 3 * m.n();
-    ws = ar.alloc<double>(8 * n3);
-    uz = ar.alloc<double>(n3);
+    ws = h->mom_buf(0, 8 * n3);
     for (int f = 0; f < 6; f++) ib_bc = ib_bc || bc.b[f] == 10;
     ib_bc = ib_bc || in.immersed == 3;
-    ul = ib_bc ? ar.alloc<double>(n3) : uz;
-    partial = ar.alloc<double>((size_t)64 * 1024);
-    red = ar.alloc<double>(128);
-    HIPCHECK(hipHostMalloc(&hpin, 128 * sizeof(double)));
-    HIPCHECK(hipHostGetDevicePointer((void**)&hpin_dev, hpin, 0));
-  }
-  ~ImplicitMomentum() {
-    if (hpin) (void)hipHostFree(hpin);
+    if (ib_bc) {
+      uz = h->mom_buf(1, n3);
+      ul = h->mom_buf(2, n3);
+    }
+    partial = h->mom_buf(3, (size_t)64 * 1024);
+    red = h->mom_buf(4, 128);
+    hpin = h->hpin + RED_MOM;
+    hpin_dev = h->hpin_dev + RED_MOM;
   }
 
-  // F(U); Uz and Ucat of U land in uz and ucat
-  void residual(const double* u, double* ucat, double* f) {
-    const dim3 grd = box_grid(m), blk(64, 4);
-    k_mm_bc_zero<<<grd, blk, 0, s>>>(m, bc, u, uz);
-    k_mm_local_ucont<<<grd, blk, 0, s>>>(m, uz, ws);
+  // f = F(u); with v, f = (F(u + h v) - f0) / h.  Ucat of U with its wall components zeroed
+  // lands in ucat
+  void residual(const double* u, double* ucat, double* f, const double* v = nullptr, double hv = 0.,
+                const double* f0 = nullptr) {
+    const unsigned grd = box_grid(m), blk = 256;
+    k_mm_local_zeroed<<<grd, blk, 0, s>>>(m, bc, u, v, hv, ib_bc ? uz : nullptr, ws);
     HIPCHECK(hipGetLastError());
     launch_c2c(s, m, d, h->met9, h->cls, h->nvert, ws, ucat, h->snap, h->grid.bctype);
     const bool bdf1 = coeff > 0.9 && coeff < 1.1;
-    k_mm_time<<<nb(), 256, 0, s>>>(n3, uz, uo, urm1 ? urm1 : uo, bdf1 ? 1 : 0, dt, f);
-    HIPCHECK(hipGetLastError());
     if (ib_bc) {
       k_mm_ib_bc<<<grd, blk, 0, s>>>(m, bc, in.immersed, in.nv, uz, ul);
       HIPCHECK(hipGetLastError());
     }
-    formfunction2(s, m, in, ul, ucat, ren, bdf1 ? 0.5 : 1.0, ws, f, true);
-    k_mm_tail<<<nb(), 256, 0, s>>>(n3, bdf1 ? rhs_o : nullptr, dp, f);
-    HIPCHECK(hipGetLastError());
+    const SnesTerms t{bc, u, v, uo, urm1 ? urm1 : uo, bdf1 ? rhs_o : nullptr, dp, f0, bdf1 ? 1 : 0, dt, hv};
+    formfunction2(s, m, in, ib_bc ? ul : nullptr, ucat, ren, bdf1 ? 0.5 : 1.0, ws, f, &t);
     evals++;
   }
 
@@ -556,12 +628,12 @@ struct ImplicitMomentum {
     const double err = std::sqrt(std::numeric_limits<double>::epsilon());
     const double t0 = now_ms();
     vfs_pp_newton_stats st{};
-    double* V = ar.alloc<double>((size_t)(M + 1) * n3);
-    double* F = ar.alloc<double>(n3);
-    double* Ft = ar.alloc<double>(n3);
-    double* Ut = ar.alloc<double>(n3);
-    double* S = ar.alloc<double>(n3);
-    double* ydev = ar.alloc<double>(M);
+    double* V = h->mom_buf(5, (size_t)(M + 1) * n3);
+    double* F = h->mom_buf(6, n3);
+    double* Ft = h->mom_buf(7, n3);
+    double* Ut = h->mom_buf(8, n3);
+    double* S = h->mom_buf(9, n3);
+    double* ydev = h->mom_buf(10, M);
     std::vector<double> H((size_t)(M + 1) * M), cs(M), sn(M), gv(M + 1), y(M);
     residual(u, ucat, F);
     double fnorm = norm(F);
@@ -596,9 +668,7 @@ struct ImplicitMomentum {
           // true residual r = -F - J s
           const double sn2 = norm(S);
           const double hfd = err * std::sqrt(1. + unorm) / sn2;
-          k_mm_axpby<<<nb(), 256, 0, s>>>(n3, u, S, hfd, Ut);
-          residual(Ut, ucat, Ft);
-          k_mm_fd<<<nb(), 256, 0, s>>>(n3, Ft, F, hfd, V);  // J s
+          residual(u, ucat, V, S, hfd, F);  // J s
           k_mm_axpby<<<nb(), 256, 0, s>>>(n3, F, V, 1., V);  // F + J s
           rnorm = norm(V);
           if (rnorm <= target) break;
@@ -613,10 +683,7 @@ struct ImplicitMomentum {
           double* vj = V + (size_t)j * n3;
           double* w = V + (size_t)(j + 1) * n3;
           const double hfd = err * std::sqrt(1. + unorm);  // |v_j| = 1
-          k_mm_axpby<<<nb(), 256, 0, s>>>(n3, u, vj, hfd, Ut);
-          residual(Ut, ucat, Ft);
-          k_mm_fd<<<nb(), 256, 0, s>>>(n3, Ft, F, hfd, w);
-          HIPCHECK(hipGetLastError());
+          residual(u, ucat, w, vj, hfd, F);  // J v_j
           for (int l = 0; l <= j; l++) H[(size_t)l * M + j] = 0.;
           for (int pass = 0; pass < 2; pass++) {  // classical Gram-Schmidt, twice
             dots(w, V, j + 1);
@@ -679,8 +746,8 @@ struct ImplicitMomentum {
     }
     st.fnorm = fnorm;
     // the solution's wall faces (implicitsolver.c:408-415) and its Ucat
-    k_mm_bc_post<<<box_grid(m), dim3(64, 4), 0, s>>>(m, bc, u);
-    k_mm_local_ucont<<<box_grid(m), dim3(64, 4), 0, s>>>(m, u, ws);
+    k_mm_bc_post<<<box_grid(m), 256, 0, s>>>(m, bc, u);
+    k_mm_local_ucont<<<box_grid(m), 256, 0, s>>>(m, u, ws);
     HIPCHECK(hipGetLastError());
     launch_c2c(s, m, d, h->met9, h->cls, h->nvert, ws, ucat, h->snap, h->grid.bctype);
     HIPCHECK(hipStreamSynchronize(s));
@@ -767,26 +834,27 @@ int vfs_pp_runge_kutta_device(vfs_pp_handle* h, const double* icsi, const double
   vfs_grid gr = h->grid;
   gr.immersed = h->immersed_ref;
   const MomIn in = make_in(&gr, met, h->nvert);
-  Arena tmp;
-  double* ws = tmp.alloc<double>(8 * M3);
-  double* pu = tmp.alloc<double>(M3);
-  double* rhs = tmp.alloc<double>(M3);
+  double* ws = h->mom_buf(0, 8 * M3);
+  double* pu = h->mom_buf(1, M3);
+  double* rhs = h->mom_buf(2, M3);
   const unsigned nb = (unsigned)((M3 + 255) / 256);
   const double alfa[4] = {0.25, 1 / 3., 0.5, 1.};
   // Contra2Cart reads Ucont with fresh whole-vector periodic ghosts (rhs.c:115-142)
   // in a local copy; the caller's ghost faces keep their values, as the
   // reference's global Ucont does
   double* lu = ws;
-  const dim3 grd = box_grid(m), blk(64, 4);
+  const unsigned grd = box_grid(m), blk = 256;
   auto contra2cart = [&]() {
     k_mm_local_ucont<<<grd, blk, 0, s>>>(m, ucont, lu);
     HIPCHECK(hipGetLastError());
     launch_c2c(s, m, h->d, h->met9, h->cls, h->nvert, lu, ucat, h->snap, h->grid.bctype);
   };
   k_mm_copy<<<nb, 256, 0, s>>>(M3, ucont, pu);
+  contra2cart();
   for (int q = 0; q < 4; q++) {
-    contra2cart();
-    formfunction2(s, m, in, ucont, ucat, ren, 1.0, ws, rhs);
+    // a stage begins with the Contra2Cart its predecessor ended with, on the same Ucont
+    if (q) launch_c2c_again(s, m, h->nvert, ucat, h->snap, h->grid.bctype);
+    formfunction2(s, m, in, nullptr, ucat, ren, 1.0, ws, rhs);  // lu holds the local Ucont
     const double a = alfa[q] * dt * st;
     k_mm_stage<<<nb, 256, 0, s>>>(M3, rhs, dp, pu, a, ucont);
     HIPCHECK(hipGetLastError());
