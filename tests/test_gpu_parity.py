@@ -656,3 +656,41 @@ def test_y_line_block_layouts(E, torch_cuda, dims):
     (a, ia), (b, ib) = outs
     assert np.linalg.norm(a - b) <= 1e-9 * np.linalg.norm(b)
     assert abs(ia - ib) <= 1
+
+
+@pytest.mark.parametrize("precision", [1, 0])
+def test_iteration_queued_ahead(E, torch_cuda, precision):
+    """The next V-cycle is queued before this iteration's scalars are read, and a zero
+    start's first iteration before ||b|| is: a zero right-hand side, every iteration
+    limit and loose and tight tolerances count iterations and V-cycles as if each were
+    waited for, and a limited solve's Phi does not depend on what was queued after it (the
+    same Phi from a restart length equal to the limit, after which nothing is queued)."""
+    torch = torch_cuda
+    c = get_case("hill_sphere")[0]
+
+    def solve(u, **kw):
+        h = handle_for(E, c, precision=precision, **kw)
+        phi = torch.zeros(c.shape, dtype=torch.float64, device="cuda")
+        st = h.poisson_solve(u, phi, c.dt, c.st, c.coeff)
+        h.close()
+        return st, phi.cpu().numpy()
+
+    u = torch.from_numpy(np.ascontiguousarray(c.fields["ucont"])).cuda()
+    st, phi = solve(torch.zeros_like(u))
+    assert st.converged and st.iterations == 0 and st.vcycles == 0 and st.rel_residual == 0.0 and not phi.any()
+    for limit in (0, 1, 2, 5):
+        st, phi = solve(u.clone(), max_iters=limit, rtol=1e-13, div_tol=0.0)
+        assert not st.converged and st.iterations == limit and st.vcycles == limit and st.bnorm > 0.0
+        if limit:
+            st2, phi2 = solve(u.clone(), max_iters=limit, restart=limit, rtol=1e-13, div_tol=0.0)
+            assert np.array_equal(phi, phi2) and st2.rel_residual == st.rel_residual
+    last = 0
+    for rtol in (0.5, 1e-2, 1e-5, 1e-9, 1e-12):
+        st, _ = solve(u.clone(), rtol=rtol, div_tol=0.0)
+        assert st.converged and st.rel_residual <= rtol and st.vcycles == st.iterations >= last
+        last = st.iterations
+    bad = u.clone()
+    bad[3, 3, 3, 0] = float("nan")
+    with pytest.raises(E.VfsPPError) as ei:
+        solve(bad)
+    assert ei.value.code == E.VFS_PP_ENONFINITE

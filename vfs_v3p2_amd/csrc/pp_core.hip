@@ -386,6 +386,31 @@ __global__ __launch_bounds__(1024) void k_finalize(const double* __restrict__ pa
   }
 }
 
+// The same sum of one vector of partials with its reciprocal (0 for 0) to inv: the squared
+// norm of a new basis vector, whose reciprocal the next Gram-Schmidt pass reads
+__global__ __launch_bounds__(1024) void k_finalize_norm(const double* __restrict__ partial, int nblk,
+                                                        double* __restrict__ out, double* __restrict__ inv,
+                                                        double* __restrict__ host) {
+  __shared__ double lds[16];
+  const int t = threadIdx.x;
+  double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
+  int b = t;
+  for (; b + 3072 < nblk; b += 4096) {
+    a0 += partial[b]; a1 += partial[b + 1024]; a2 += partial[b + 2048]; a3 += partial[b + 3072];
+  }
+  for (; b < nblk; b += 1024) a0 += partial[b];
+  a0 = wave_sum((a0 + a1) + (a2 + a3));
+  if ((t & 63) == 0) lds[t >> 6] = a0;
+  __syncthreads();
+  if (t == 0) {
+    double s = lds[0];
+    for (int w = 1; w < 16; w++) s += lds[w];
+    out[0] = s;
+    inv[0] = s > 0. ? 1. / s : 0.;
+    host[0] = s;
+  }
+}
+
 template <int NV>
 __global__ __launch_bounds__(256) void k_multidot(size_t n, const double* __restrict__ w, const double* __restrict__ V,
                                                   size_t ldv, double* __restrict__ partial, int nblk) {
@@ -768,6 +793,11 @@ void launch_divergence(hipStream_t s, Dmda m, Dims d, const uint32_t* code, cons
 void launch_finalize(hipStream_t s, const double* partial, int nvec, int nblk, double* out, int op,
                      double* host_mirror) {
   k_finalize<<<nvec, 1024, 0, s>>>(partial, nblk, out, op, host_mirror);
+  HIPCHECK(hipGetLastError());
+}
+
+void launch_finalize_norm(hipStream_t s, const double* partial, int nblk, double* out, double* inv, double* host) {
+  k_finalize_norm<<<1, 1024, 0, s>>>(partial, nblk, out, inv, host);
   HIPCHECK(hipGetLastError());
 }
 

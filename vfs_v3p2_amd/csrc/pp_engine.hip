@@ -375,10 +375,28 @@ void need_partials(vfs_pp_handle* h, size_t nvec, size_t nblk) {
                                          std::to_string(h->partial_cap) + ")");
 }
 
+// A solve that starts from zero needs no residual check before its first cycle (r = b,
+// and ||b|| <= rtol ||b|| cannot hold), so its first iteration is queued behind the
+// right-hand side without waiting for ||b||.
+static bool starts_unchecked(const vfs_pp_handle* h) {
+  return h->opts.zero_guess != 0 && h->opts.orthog == 2 && h->opts.rtol < 1. && h->opts.max_iters > 0;
+}
+
+void solve_start_stats(vfs_pp_handle* h, vfs_pp_stats* S);
+
 // FGMRES(m) with CGS2; right preconditioner = one V-cycle.  Solves A x = b
-// (x holds the initial guess).  Returns iterations; fills rel.
+// (x holds the initial guess).  Returns iterations; fills rel.  With starts_unchecked
+// the prologue is still on the stream: S's right-hand-side figures are read with the
+// first iteration's.
+//
+// With the lazily normalised basis (orthog 2) nothing the next V-cycle reads comes from
+// the host, so where the residual estimate says that another iteration will be needed
+// (even at a third of the best reduction seen), its V-cycle is queued before the host
+// waits for this iteration's scalars: the device has no gap of a host round trip, about
+// 15 us per iteration.  A V-cycle queued in vain only writes its own buffers.
 template <typename TZ>
-static int fgmres(vfs_pp_handle* h, double bnorm, double* rel_out, int* vcyc, bool* conv) {
+static int fgmres(vfs_pp_handle* h, vfs_pp_stats* S, double* rel_out, int* vcyc, bool* conv) {
+  double bnorm = S->bnorm;
   const size_t n = h->d.n();
   const int m = h->mrest;
   const double rtol = h->opts.rtol;
@@ -396,18 +414,30 @@ static int fgmres(vfs_pp_handle* h, double bnorm, double* rel_out, int* vcyc, bo
   double tgt = rtol * bnorm;
   // the first check of a zero-start solve needs no operator pass (r = b)
   bool x_zero = h->opts.zero_guess != 0;
+  bool unread = starts_unchecked(h);  // ||b|| is not on the host yet
+  double best_ratio = 1e-3;           // of successive residual estimates; a guess before the first
+  auto queue_vcycle = [&](int j) {
+    // z_j = M^-1 v_j (the V-cycle reads v_j from its level-0 right-hand side)
+    h->mg->set_out(Z + (size_t)j * n);
+    h->mg->tail = (h->opts.fused & 1) != 0;
+    h->mg->use_fd = fd0 != nullptr;
+    h->mg->vcycle(h->s);
+  };
   while (true) {
     int nb = 0;  // block count of the reductions below
-    launch_true_residual(h, h->s, x_zero);
-    HIPCHECK(hipStreamSynchronize(h->s));
-    const double beta = std::sqrt(true_residual_host_norm2(h, x_zero));
-    rel = bnorm > 0. ? beta / bnorm : 0.;
-    if (!std::isfinite(beta)) throw StatusError(VFS_PP_ENONFINITE, "non-finite residual");
-    if (h->opts.verbose)
-      std::fprintf(stderr, "vfs_pp: restart at it %d  true rel %.3e  div est %.3e\n", it, rel,
-                   h->div_fac * h->hpin[RED_DIVEST]);
-    if (residual_verdict(h, beta, bnorm, tgt)) { *conv = true; break; }
-    if (it >= h->opts.max_iters) break;
+    double beta = 0.;
+    if (!unread) {
+      launch_true_residual(h, h->s, x_zero);
+      HIPCHECK(hipStreamSynchronize(h->s));
+      beta = std::sqrt(true_residual_host_norm2(h, x_zero));
+      rel = bnorm > 0. ? beta / bnorm : 0.;
+      if (!std::isfinite(beta)) throw StatusError(VFS_PP_ENONFINITE, "non-finite residual");
+      if (h->opts.verbose)
+        std::fprintf(stderr, "vfs_pp: restart at it %d  true rel %.3e  div est %.3e\n", it, rel,
+                     h->div_fac * h->hpin[RED_DIVEST]);
+      if (residual_verdict(h, beta, bnorm, tgt)) { *conv = true; break; }
+      if (it >= h->opts.max_iters) break;
+    }
     // v_0 = r / beta and its copy as the first V-cycle input
     launch_scale_conv<TZ>(h->s, n, true_residual_src(h, x_zero), true_residual_norm2(h, x_zero), h->V,
                           static_cast<TZ*>(h->mg->f0()), dinv0, fd0);
@@ -415,19 +445,16 @@ static int fgmres(vfs_pp_handle* h, double bnorm, double* rel_out, int* vcyc, bo
     if (h->opts.orthog == 2) {
       nu[0] = 1.;
       sigma[0] = 1.;
-      h->hpin[RED_NUINV2] = 1.;
-      h2d(h->s, h->red + RED_NUINV2, h->hpin + RED_NUINV2, 1);
+      launch_fill(h->s, 1, h->red + RED_NUINV2, 1.);
     }
     std::fill(gv.begin(), gv.end(), 0.);
     gv[0] = beta;
     int j = 0;
+    bool queued = false;  // V-cycle j is on the stream already
     for (; j < m && it < h->opts.max_iters; j++) {
       double* w = h->V + (size_t)(j + 1) * n;
-      // z_j = M^-1 v_j (the V-cycle reads v_j from its level-0 right-hand side)
-      h->mg->set_out(Z + (size_t)j * n);
-      h->mg->tail = (h->opts.fused & 1) != 0;
-      h->mg->use_fd = fd0 != nullptr;
-      h->mg->vcycle(h->s);
+      if (!queued) queue_vcycle(j);
+      queued = false;
       (*vcyc)++;
       double sub = 0.;
       if (h->opts.orthog == 2) {
@@ -441,8 +468,29 @@ static int fgmres(vfs_pp_handle* h, double bnorm, double* rel_out, int* vcyc, bo
         launch_finalize(h->s, h->partial, nv + 1, nb, h->red + 8, 0, h->hpin_dev + 8);
         launch_axpy_norm<TZ>(h->s, n, w, h->V, n, nv, h->red + 8, h->red + RED_NUINV2, h->red + 8 + nv,
                              static_cast<TZ*>(h->mg->f0()), h->partial, &nb, dinv0, fd0);
-        launch_finalize(h->s, h->partial, 1, nb, h->red, 0, h->hpin_dev);
-        HIPCHECK(hipStreamSynchronize(h->s));
+        launch_finalize_norm(h->s, h->partial, nb, h->red, h->red + RED_NUINV2 + j + 1, h->hpin_dev);
+        if (j + 1 < m && it + 1 < h->opts.max_iters &&
+            (unread ? best_ratio > rtol : std::fabs(gv[j]) * best_ratio > tgt)) {
+          HIPCHECK(hipEventRecord(h->ev, h->s));
+          queue_vcycle(j + 1);
+          queued = true;
+          HIPCHECK(hipEventSynchronize(h->ev));
+        } else {
+          HIPCHECK(hipStreamSynchronize(h->s));
+        }
+        if (unread) {
+          unread = false;
+          solve_start_stats(h, S);
+          bnorm = S->bnorm;
+          tgt = rtol * bnorm;
+          if (bnorm == 0.) {
+            *vcyc = 0;
+            *conv = true;
+            *rel_out = 0.;
+            return 0;
+          }
+          gv[0] = bnorm;
+        }
         const double a2 = h->hpin[8 + nv];
         double b2 = h->hpin[0];
         for (int l = 0; l <= j; l++) H[(size_t)l * m + j] = h->hpin[8 + l] / (nu[l] * sigma[j]);
@@ -451,16 +499,15 @@ static int fgmres(vfs_pp_handle* h, double bnorm, double* rel_out, int* vcyc, bo
           launch_finalize(h->s, h->partial, nv, nb, h->red + 72, 0, h->hpin_dev + 72);
           launch_axpy_norm<TZ>(h->s, n, w, h->V, n, nv, h->red + 72, h->red + RED_NUINV2, h->red + 8 + nv,
                                static_cast<TZ*>(h->mg->f0()), h->partial, &nb, dinv0, fd0);
-          launch_finalize(h->s, h->partial, 1, nb, h->red, 0, h->hpin_dev);
+          launch_finalize_norm(h->s, h->partial, nb, h->red, h->red + RED_NUINV2 + j + 1, h->hpin_dev);
           HIPCHECK(hipStreamSynchronize(h->s));
           for (int l = 0; l <= j; l++) H[(size_t)l * m + j] += h->hpin[72 + l] / (nu[l] * sigma[j]);
           b2 = h->hpin[0];
+          queued = false;  // the V-cycle's input has changed
         }
         nu[j + 1] = std::sqrt(b2);
         sigma[j + 1] = host_conv_scale(a2) * nu[j + 1];
         sub = nu[j + 1] / sigma[j];
-        h->hpin[RED_NUINV2 + j + 1] = b2 > 0. ? 1. / b2 : 0.;
-        h2d(h->s, h->red + RED_NUINV2 + j + 1, h->hpin + RED_NUINV2 + j + 1, 1);
       } else if (h->opts.orthog == 1) {
         // two-pass classical Gram-Schmidt (CGS2)
         launch_apply64<TZ>(h->s, h->d, h->g64, h->code, Z + (size_t)j * n, w, false);
@@ -510,6 +557,9 @@ static int fgmres(vfs_pp_handle* h, double bnorm, double* rel_out, int* vcyc, bo
       gv[j + 1] = -sn[j] * gv[j];
       gv[j] = cs[j] * gv[j];
       it++;
+      // a third of the best reduction of one iteration so far (a first one may be small)
+      const double ratio = gv[j] == 0. && gv[j + 1] == 0. ? 1. : std::fabs(gv[j + 1]) / std::hypot(gv[j], gv[j + 1]);
+      best_ratio = j == 0 ? ratio / 3. : std::min(best_ratio, ratio / 3.);
       if (!std::isfinite(gv[j + 1])) throw StatusError(VFS_PP_ENONFINITE, "non-finite Krylov residual");
       if (h->opts.verbose)
         std::fprintf(stderr, "vfs_pp: it %3d  est rel %.3e  h_jj %.3e  sub %.3e\n", it, std::fabs(gv[j + 1]) / bnorm,
@@ -677,28 +727,36 @@ void solve_epilogue(vfs_pp_handle* h, double* phi, vfs_pp_stats* S) {
 
 static double phi_mean_of(const vfs_pp_handle* h) { return h->n_lt > 0. ? h->hpin[RED_MEAN] / h->n_lt : 0.; }
 
+// VolumeFlux to Convert_Phi2_Phi.  With wait = false the epilogue is left on the stream and
+// S's phi_mean (phi_mean_of after the next sync) and ms_total to the caller.
 static void poisson_solve(vfs_pp_handle* h, double* ucont, double* phi, double dt, double st, double coeff,
-                          vfs_pp_stats* out) {
+                          vfs_pp_stats* out, bool wait) {
   const double t0 = now_ms();
   vfs_pp_stats S{};
   solve_prologue(h, ucont, dt, st, coeff);
-  HIPCHECK(hipStreamSynchronize(h->s));
-  solve_start(h, phi, &S);
+  if (starts_unchecked(h)) {
+    launch_fill(h->s, h->d.n(), h->x, 0.);
+  } else {
+    HIPCHECK(hipStreamSynchronize(h->s));
+    solve_start(h, phi, &S);
+  }
   double rel = 0.;
   int vc = 0;
   bool conv = false;
   int it;
-  if (S.bnorm == 0.) { it = 0; rel = 0.; conv = true; }
-  else if (h->opts.precision == 1) it = fgmres<float>(h, S.bnorm, &rel, &vc, &conv);
-  else it = fgmres<double>(h, S.bnorm, &rel, &vc, &conv);
+  if (!starts_unchecked(h) && S.bnorm == 0.) { it = 0; rel = 0.; conv = true; }
+  else if (h->opts.precision == 1) it = fgmres<float>(h, &S, &rel, &vc, &conv);
+  else it = fgmres<double>(h, &S, &rel, &vc, &conv);
   S.iterations = it;
   S.vcycles = vc;
   S.rel_residual = rel;
   S.converged = conv ? 1 : 0;
   solve_epilogue(h, phi, &S);
-  HIPCHECK(hipStreamSynchronize(h->s));
-  S.phi_mean = phi_mean_of(h);
-  S.ms_total = now_ms() - t0;
+  if (wait) {
+    HIPCHECK(hipStreamSynchronize(h->s));
+    S.phi_mean = phi_mean_of(h);
+    S.ms_total = now_ms() - t0;
+  }
   if (out) *out = S;
 }
 
@@ -848,6 +906,10 @@ int vfs_pp_create(const vfs_grid* g, const vfs_pp_opts* o, vfs_pp_handle** out) 
   // legacy default stream (PyTorch's default stream, for one) and before work
   // queued there afterwards, so inputs written just before a call are seen
   HIPCHECK(hipStreamCreateWithFlags(&h->s, hipStreamDefault));
+  if (hipEventCreateWithFlags(&h->ev, hipEventDisableTiming) != hipSuccess) {
+    (void)hipStreamDestroy(h->s);
+    throw StatusError(VFS_PP_EHIP, "event creation failed");
+  }
   *out = h.release();
   return VFS_PP_OK;
   ABI_END
@@ -860,6 +922,7 @@ int vfs_pp_destroy(vfs_pp_handle* h) {
   h->mg.reset();
   h->ar.release();
   if (h->hpin) (void)hipHostFree(h->hpin);
+  if (h->ev) (void)hipEventDestroy(h->ev);
   if (h->s) (void)hipStreamDestroy(h->s);
   delete h;
   return VFS_PP_OK;
@@ -959,7 +1022,7 @@ int vfs_pp_poisson_solve_device(vfs_pp_handle* h, double* ucont, double* phi, do
   if (!h || !ucont || !phi || !(dt > 0.) || coeff == 0.) return VFS_PP_EINVAL;
   ensure_unbound(h);
   vfs_pp_stats S{};
-  poisson_solve(h, ucont, phi, dt, st, coeff, &S);
+  poisson_solve(h, ucont, phi, dt, st, coeff, &S, true);
   if (stats) *stats = S;
   return S.converged ? VFS_PP_OK : VFS_PP_ENOCONV;
   ABI_END
@@ -1002,10 +1065,11 @@ int vfs_pp_project_device(vfs_pp_handle* h, double* ucont, double* phi, double* 
   ensure_unbound(h);
   const double t0 = now_ms();
   vfs_pp_stats S{};
-  poisson_solve(h, ucont, phi, dt, st, coeff, &S);
+  poisson_solve(h, ucont, phi, dt, st, coeff, &S, false);
   update_pressure(h, p, phi);
   projection(h, ucont, phi, ucat, dt, st, coeff);
-  S.max_div = divergence(h, ucont);
+  S.max_div = divergence(h, ucont);  // waits for the stream
+  S.phi_mean = phi_mean_of(h);
   S.ms_total = now_ms() - t0;
   bool ok = S.converged;
   if (h->opts.div_tol > 0. && !(S.max_div <= h->opts.div_tol)) ok = false;

@@ -379,6 +379,7 @@ struct vfs_pp_handle {
   pp::Dmda m{};
   pp::Dims d{};
   hipStream_t s = nullptr;
+  hipEvent_t ev = nullptr;  // this iteration's scalars are on the host (fgmres)
   pp::Arena ar;   // buffers sized by the grid alone
   pp::Arena geo;  // buffers of the current geometry (hierarchy, face list), renewed by each set-up
   pp::Arena setup_tmp;  // set-up scratch, kept between set-ups of a moving body

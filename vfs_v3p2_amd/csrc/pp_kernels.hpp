@@ -137,6 +137,8 @@ void launch_divergence(hipStream_t s, Dmda m, Dims d, const uint32_t* code, cons
 // out[v] = sum_b partial[v*nblk + b] in a fixed order (deterministic); op 0 sum, 1 max
 void launch_finalize(hipStream_t s, const double* partial, int nvec, int nblk, double* out, int op,
                      double* host_mirror = nullptr);
+// one vector's sum, its reciprocal (0 for 0) to inv and the host mirror
+void launch_finalize_norm(hipStream_t s, const double* partial, int nblk, double* out, double* inv, double* host);
 void launch_multidot(hipStream_t s, size_t n, const double* w, const double* V, size_t ldv, int nv, double* partial,
                      int* nblk);
 void launch_axpy_multi(hipStream_t s, size_t n, double* w, const double* V, size_t ldv, int nv, const double* h,
