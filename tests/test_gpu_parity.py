@@ -628,7 +628,8 @@ def test_y_line_layouts_against_the_oracle(E, torch_cuda, precision, ny):
 
 
 @pytest.mark.parametrize("dims", [(7, 64, 5), (21, 65, 3), (9, 129, 7), (17, 256, 3), (96, 33, 90), (128, 65, 67),
-                                  (70, 130, 66), (130, 131, 127), (3, 40, 5)])
+                                  (70, 130, 66), (130, 131, 127), (3, 40, 5), (130, 193, 128),
+                                  (91, 225, 91)])
 def test_y_line_block_layouts(E, torch_cuda, dims):
     """Every block layout of the segmented y-line step (line_layout: chosen by line
     length and line count, differently in FP32 and FP64), at odd sizes that leave

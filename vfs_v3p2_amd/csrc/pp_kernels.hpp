@@ -215,8 +215,11 @@ HD inline bool line_seg_fits(const Dims& d) {
 // The bounds are where the measured step times cross, in us (narrow / middle / wide):
 // FP32 64x64x64 6.4 / 7.2 / 9.5, 256x64x256 37.4 / 37.3 / 41.2, 64x100x64 - / 9.0 / 12.2,
 // 100x110x100 - / 20.5 / 15.8, 64x200x32 10.9 / 18.3 / 20.4, 128x256x64 21.7 / 20.5 / 27.3,
-// 512x256x256 394 / 384 / 375; FP64 64x100x64 15.5 / - / 31.1, 131x77x93 44.0 / - / 28.9,
-// 100x200x100 69.3 / 75.4 / -.
+// 512x256x256 394 / 384 / 375; FP64 64x100x64 15.5 / - / 31.1, 131x77x93 44.0 / - / 28.9.
+// FP64 lines of more than 128 rows (8 x 8 x 16 / 12 x 4 x 16 / 8 x 16 x 32 / 16 x 8 x 32 rows
+// x waves x lanes): 256x150x200 332 / 278 / 285 / 306, 100x200x100 69.3 / - / 82.7 / 80.0,
+// 256x200x128 247 / - / 232 / 237, 128x256x64 65.9 / - / 51.6 / 49.0, 512x256x256 1141 / - /
+// 1119 / 1098.
 constexpr int LINE_LAYOUTS = 7;
 template <typename T>
 inline int line_layout(int ny, size_t lines) {
@@ -226,7 +229,10 @@ inline int line_layout(int ny, size_t lines) {
     return lines < 4096 ? 4 : lines < 16384 ? 5 : 6;
   }
   if (ny <= 64) return 0;
-  return ny <= 128 && lines >= 8192 ? 2 : 1;
+  if (ny <= 128) return lines < 8192 ? 1 : 2;
+  if (ny <= 192) return lines < 8192 ? 1 : 3;
+  if (ny <= 224) return lines < 16384 ? 1 : 4;
+  return lines < 8192 ? 1 : 5;
 }
 
 // Chebyshev smoothing launch modes (see smooth_point_cell); SM_POWER is one step

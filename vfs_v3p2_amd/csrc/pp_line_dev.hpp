@@ -182,7 +182,10 @@ inline void with_line_layout(int y, F&& fn) {
     switch (y) {
       case 0: fn(LineLayout<4, 4, 16, 2>{}); break;
       case 1: fn(LineLayout<8, 8, 16, 0>{}); break;
-      default: fn(LineLayout<8, 16, 64, 0>{});
+      case 2: fn(LineLayout<8, 16, 64, 0>{}); break;
+      case 3: fn(LineLayout<12, 4, 16, 0>{}); break;
+      case 4: fn(LineLayout<8, 16, 32, 0>{}); break;
+      default: fn(LineLayout<16, 8, 32, 0>{});
     }
   }
 }
