@@ -695,3 +695,38 @@ def test_iteration_queued_ahead(E, torch_cuda, precision):
     with pytest.raises(E.VfsPPError) as ei:
         solve(bad)
     assert ei.value.code == E.VFS_PP_ENONFINITE
+
+
+@pytest.mark.parametrize("dims", [(3, 150, 150), (65, 34, 33), (127, 23, 25), (129, 33, 17), (130, 256, 3),
+                                  (259, 191, 3), (40, 41, 39)])
+def test_pair_walk(E, torch_cuda, dims):
+    """The FP64 operator with two cells per thread (levels of 65536 cells on): rows shorter
+    than a wave, odd rows whose last pair overlaps the one before, rows of one wave of
+    pairs and one more, planes walked in slabs with a short last one, and one grid below
+    the bound.  The converged Phi has to satisfy the system in the coefficient form, which
+    shares none of that code: |b - A Phi| <= 1e-11 |b| from a true residual of 1e-12 |b|,
+    with the rounding of a 19-term row on top (the two forms' rows differ by at most
+    38 eps |A| |Phi|, far below 1e-11 |b| at these sizes)."""
+    torch = torch_cuda
+    nx, ny, nz = dims
+    c = (cases.hill_case(nx, ny, nz, h=0.2, beta=1.5, sphere=(0.6, 0.9, 0.0, 0.25), seed=8) if nx > 100 and nz > 3
+         else cases.channel_case(nx, ny, nz, beta=1.5, seed=8))
+    print(f"pair walk: {c.name}", flush=True)
+    A = O.Assembled(c, drop=False)
+    for precision in (0, 1):
+        h = handle_for(E, c, precision=precision, rtol=1e-12, div_tol=0.0, max_iters=400)
+        u = torch.from_numpy(np.ascontiguousarray(c.fields["ucont"])).cuda()
+        phi = torch.zeros(c.shape, dtype=torch.float64, device="cuda")
+        st = h.poisson_solve(u, phi, c.dt, c.st, c.coeff, strict=True)
+        for ax, per in zip((2, 1, 0), c.per):  # the periodic images apply() reads
+            if per:
+                phi.select(ax, 0).copy_(phi.select(ax, -2))
+                phi.select(ax, -1).copy_(phi.select(ax, 1))
+        y = torch.zeros_like(phi)
+        h.apply(phi, y)
+        h.close()
+        b = O.rhs(A.g, u.cpu().numpy(), A.nvert, c.dt, c.st, c.coeff)
+        r = np.abs(y.cpu().numpy() - b)[A.fluid_cells]
+        bn = np.linalg.norm(b[A.fluid_cells])
+        assert st.converged and abs(st.bnorm - bn) <= 1e-12 * bn
+        assert np.linalg.norm(r) <= 1e-11 * bn

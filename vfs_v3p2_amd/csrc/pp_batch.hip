@@ -75,15 +75,8 @@ using SlotDev = int2;
 // Cells of an item are walked flat, 256 consecutive cells per tile (i fastest),
 // so a level narrower than a wave still fills every lane.  Returns false past the
 // last cell.
-__device__ __forceinline__ bool flat_cell(const Dims& d, uint32_t lt, int& i, int& j, int& k) {
-  const uint32_t e = lt * 256u + threadIdx.x + 64u * threadIdx.y;
-  const uint32_t nxy = (uint32_t)d.nx * (uint32_t)d.ny;
-  if (e >= nxy * (uint32_t)d.nz) return false;
-  k = (int)(e / nxy);
-  const uint32_t r = e - (uint32_t)k * nxy;
-  j = (int)(r / (uint32_t)d.nx);
-  i = (int)(r - (uint32_t)j * (uint32_t)d.nx);
-  return true;
+__device__ __forceinline__ bool flat_tile_cell(const Dims& d, uint32_t lt, int& i, int& j, int& k) {
+  return flat_cell(d, lt * 256u + threadIdx.x + 64u * threadIdx.y, i, j, k);
 }
 
 // Tile shapes of the cell walk, chosen per launch by the autotuner: 0 walks 256
@@ -98,7 +91,7 @@ HDI uint32_t shape_tiles(int shape, const Dims& d) {
   return (((uint32_t)d.nx + tx - 1) >> lw) * (((uint32_t)d.ny + ty - 1) / ty) * (uint32_t)d.nz;
 }
 __device__ __forceinline__ bool shaped_cell(int shape, const Dims& d, uint32_t lt, int& i, int& j, int& k) {
-  if (shape == 0) return flat_cell(d, lt, i, j, k);
+  if (shape == 0) return flat_tile_cell(d, lt, i, j, k);
   const uint32_t lw = shape_log2_tx(shape), tx = 1u << lw, ty = 256u >> lw;
   const uint32_t e = threadIdx.x + 64u * threadIdx.y;
   const uint32_t nti = ((uint32_t)d.nx + tx - 1) >> lw, ntj = ((uint32_t)d.ny + ty - 1) / ty;
@@ -182,7 +175,6 @@ struct ApplyItem {
   double* V;
   size_t n;
   int slot;
-  uint32_t tx, ty;
 };
 
 template <typename T>
@@ -345,8 +337,8 @@ __global__ __launch_bounds__(256) void kb_dense(const DenseItem<T>* __restrict__
 
 // w = A z_j (FP64 flux form) into V_{j+1}; per-wave partial sums of w.V_l (l <= j)
 // and w.w at partial[l * 4 total + 4 t + wave]
-template <typename T>
-__global__ __launch_bounds__(256) void kb_apply_dots(const ApplyItem<T>* __restrict__ items,
+template <typename T, bool PAIRS>
+__global__ __launch_bounds__(256, 3) void kb_apply_dots(const ApplyItem<T>* __restrict__ items,
                                                      const uint32_t* __restrict__ start, int nitems, uint32_t total,
                                                      const SlotDev* __restrict__ sd, double* __restrict__ partial) {
   FOR_TILES(total, t) {
@@ -355,15 +347,9 @@ __global__ __launch_bounds__(256) void kb_apply_dots(const ApplyItem<T>* __restr
     const ApplyItem<T>& I = items[q];
     const SlotDev st = sd[tw_ & 0xffffu];
     if (!st.y) continue;
-    int i = 0, j = 0, k = 0;
-    const bool in = flat_cell(I.d, t - start[q], i, j, k);
-    const T* z = I.Z + (size_t)st.x * I.n;
-    double* w = I.V + (size_t)(st.x + 1) * I.n;
-    const size_t c = in ? I.d.idx(i, j, k) : 0;
-    double v8[8];
-    wave_dots_prefetch(in, c, I.V, I.n, st.x + 1, v8);
-    const double wv = in ? apply_cell(I.d, I.g, I.code, z, w, i, j, k) : 0.;
-    wave_dots(in, c, wv, I.V, I.n, st.x + 1, v8, partial, 4 * (size_t)total, 4 * (size_t)t + threadIdx.y);
+    apply_dots<PAIRS>(I.d, pair_slab(I.d), (t - start[q]) * 256u + threadIdx.x, I.g, I.code,
+                      I.Z + (size_t)st.x * I.n, I.V + (size_t)(st.x + 1) * I.n, I.V, I.n, st.x + 1, partial,
+                      4 * (size_t)total, 4 * (size_t)t + (threadIdx.x >> 6));
   }
 }
 
@@ -606,18 +592,18 @@ __global__ __launch_bounds__(256) void kb_phase(const PhaseItem* __restrict__ it
       if (in) ibflux_correct_face(I.faces[e], I.w0, I.i0, I.sc);
     } else if constexpr (OP == PH_RHS) {
       double v = 0.;
-      if (flat_cell(I.d, lt, i, j, k)) v = rhs_cell(I.m, I.d, I.r0, I.cls, I.s0, I.w0, i, j, k);
+      if (flat_tile_cell(I.d, lt, i, j, k)) v = rhs_cell(I.m, I.d, I.r0, I.cls, I.s0, I.w0, i, j, k);
       v = block_sum(v, lds);
       if (threadIdx.x == 0) partial[t] = v;
     } else if constexpr (OP == PH_GATHER) {
-      if (flat_cell(I.d, lt, i, j, k)) gather_phi_cell(I.m, I.d, I.r0, I.cls, I.w0, i, j, k);
+      if (flat_tile_cell(I.d, lt, i, j, k)) gather_phi_cell(I.m, I.d, I.r0, I.cls, I.w0, i, j, k);
     } else if constexpr (OP == PH_ZERO) {
       if (in) I.w0[e] = 0.;
     } else if constexpr (OP == PH_UPDATE_X) {
       if (in) update_x_elem(I.w0, static_cast<const T*>(I.z), I.ld, I.i0, I.sc, e);
     } else if constexpr (OP == PH_RESID) {
       double v = 0.;
-      if (flat_cell(I.d, lt, i, j, k)) v = residual_cell<double>(I.d, I.g, I.code, I.r0, I.r1, I.w0, i, j, k);
+      v = residual_at<true>(I.d, pair_slab(I.d), e, I.g, I.code, I.r0, I.r1, I.w0);
       v = block_sum(v, lds);
       if (threadIdx.x == 0) partial[t] = v;
     } else if constexpr (OP == PH_DIVEST) {
@@ -637,26 +623,26 @@ __global__ __launch_bounds__(256) void kb_phase(const PhaseItem* __restrict__ it
         if (I.cls[e] & CLS_LT) I.w0[e] += val;
       }
     } else if constexpr (OP == PH_SCATTER) {
-      if (flat_cell(I.d, lt, i, j, k)) scatter_cell(I.m, I.d, I.r0, I.cls, I.w0, nullptr, i, j, k);
+      if (flat_tile_cell(I.d, lt, i, j, k)) scatter_cell(I.m, I.d, I.r0, I.cls, I.w0, nullptr, i, j, k);
     } else if constexpr (OP == PH_PERIODIC) {
       if (in && boundary_point(I.m, e, i, j, k)) periodic_point(I.m, I.w0, I.i0, i, j, k);
     } else if constexpr (OP == PH_ADD_PHI) {
-      if (flat_cell(I.d, lt, i, j, k)) add_phi_cell(I.m, I.d, I.cls, I.r0, I.w0, i, j, k);
+      if (flat_tile_cell(I.d, lt, i, j, k)) add_phi_cell(I.m, I.d, I.cls, I.r0, I.w0, i, j, k);
     } else if constexpr (OP == PH_PROJECTION) {
-      if (flat_cell(I.d, lt, i, j, k)) projection_cell(I.m, I.d, I.g, I.code, I.cls, I.r0, I.w0, I.s0, i, j, k);
+      if (flat_tile_cell(I.d, lt, i, j, k)) projection_cell(I.m, I.d, I.g, I.code, I.cls, I.r0, I.w0, I.s0, i, j, k);
     } else if constexpr (OP == PH_UCONT_GHOSTS) {
       if (in && boundary_point(I.m, e, i, j, k)) ucont_ghost_point(I.m, I.w0, i, j, k);
     } else if constexpr (OP == PH_C2C_CORE) {
-      if (flat_cell(I.d, lt, i, j, k)) c2c_core_cell(I.m, I.d, I.r0, I.cls, I.r1, I.w0, i, j, k);
+      if (flat_tile_cell(I.d, lt, i, j, k)) c2c_core_cell(I.m, I.d, I.r0, I.cls, I.r1, I.w0, i, j, k);
     } else if constexpr (OP == PH_VEC_GHOSTS) {
       if (in && boundary_point(I.m, e, i, j, k)) vec_ghost_point(I.m, I.w0, I.w1, i, j, k);
     } else if constexpr (OP == PH_C2C_BC) {
       if (in && boundary_point(I.m, e, i, j, k)) c2c_bc_point(I.m, I.r0, I.r1, I.w0, I.bc, i, j, k);
     } else if constexpr (OP == PH_C2C_SOLID) {
-      if (flat_cell(I.d, lt, i, j, k)) c2c_solid_cell(I.m, I.d, I.cls, I.w0, i, j, k);
+      if (flat_tile_cell(I.d, lt, i, j, k)) c2c_solid_cell(I.m, I.d, I.cls, I.w0, i, j, k);
     } else if constexpr (OP == PH_DIVERGENCE) {
       double v = 0.;
-      if (flat_cell(I.d, lt, i, j, k)) v = divergence_cell(I.m, I.d, I.code, I.r0, I.r1, i, j, k);
+      if (flat_tile_cell(I.d, lt, i, j, k)) v = divergence_cell(I.m, I.d, I.code, I.r0, I.r1, i, j, k);
       v = block_max(v, lds);
       if (threadIdx.x == 0) partial[t] = v;
     }
@@ -1097,6 +1083,9 @@ struct BatchCore {
       std::vector<FinItem> fa, fv;
       uint32_t ta = 0, tv = 0;
       int mmax = 1;
+      size_t cells = 0;
+      for (int q : mem) cells += slots[q].h->d.n();
+      const bool pairs = takes_pairs(cells);
       for (int q : mem) {
         vfs_pp_handle* h = slots[q].h;
         const size_t n = h->d.n();
@@ -1108,9 +1097,7 @@ struct BatchCore {
         a.V = h->V;
         a.n = n;
         a.slot = q;
-        a.tx = (uint32_t)(h->d.nx + 63) / 64;
-        a.ty = (uint32_t)(h->d.ny + 3) / 4;
-        const uint32_t na = cell_tiles(h->d);
+        const uint32_t na = pairs ? (pair_count(h->d) + 255) / 256 : cell_tiles(h->d);
         fa.push_back(FinItem{h->red, h->hpin_dev, ta, ta + na, q});
         ta += na;
         ai.push_back(a);
@@ -1139,7 +1126,7 @@ struct BatchCore {
       for (size_t q = 0; q < vi.size(); q++) { sv[q] = acc; acc += vn[q]; }
       auto pa = upload(ai, sa, ta);
       auto pv = upload(vi, sv, tv);
-      apply = Launch{K_APPLY, 0, pa.first, pa.second, (int)ai.size(), ta, 2048};
+      apply = Launch{K_APPLY, pairs ? 1 : 0, pa.first, pa.second, (int)ai.size(), ta, 2048};
       axd = Launch{K_AXD, 0, pv.first, pv.second, (int)vi.size(), tv, 2048};
       axs = Launch{K_AXS, 0, pv.first, pv.second, (int)vi.size(), tv, 2048};
       axn = Launch{K_AXN, 0, pv.first, pv.second, (int)vi.size(), tv, 2048};
@@ -1265,8 +1252,12 @@ struct BatchCore {
         kb_dense<T><<<W, 256, 0, s>>>(static_cast<const DenseItem<T>*>(L.items), L.start, L.nitems, L.total, sd);
         break;
       case K_APPLY:
-        kb_apply_dots<T><<<W, dim3(64, 4, 1), 0, s>>>(static_cast<const ApplyItem<T>*>(L.items), L.start, L.nitems,
-                                                      L.total, sd, partial);
+        if (L.mode)
+          kb_apply_dots<T, true><<<W, 256, 0, s>>>(static_cast<const ApplyItem<T>*>(L.items), L.start, L.nitems,
+                                                   L.total, sd, partial);
+        else
+          kb_apply_dots<T, false><<<W, 256, 0, s>>>(static_cast<const ApplyItem<T>*>(L.items), L.start, L.nitems,
+                                                    L.total, sd, partial);
         break;
       case K_AXD:
         kb_axpy_dots<T><<<W, 256, 0, s>>>(static_cast<const VecItem<T>*>(L.items), L.start, L.nitems, L.total, sd,
@@ -1718,6 +1709,7 @@ struct BatchCore {
         vfs_pp_handle* h = slots[q].h;
         if (slots[q].x_zero) continue;
         PhaseItem it = case_item(h);
+        it.n = pair_count(h->d);
         it.r0 = h->b;
         it.r1 = h->x;
         it.w0 = h->r;

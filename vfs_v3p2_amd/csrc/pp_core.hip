@@ -16,6 +16,10 @@ namespace pp {
 
 namespace {
 
+// blocks of a flat walk, by pairs or by cells
+inline unsigned walk_blocks(const Dims& d, bool pairs) {
+  return (unsigned)(((pairs ? (size_t)pair_count(d) : d.n()) + 255) / 256);
+}
 inline dim3 cell_grid(const Dims& d) { return dim3((d.nx + 63) / 64, (d.ny + 3) / 4, d.nz); }
 inline dim3 dmda_grid(const Dmda& m) { return dim3((m.mx + 63) / 64, (m.my + 3) / 4, m.mz); }
 inline unsigned bnd_blocks(const Dmda& m) { return (boundary_count(m) + 255u) / 256u; }
@@ -117,47 +121,56 @@ __global__ __launch_bounds__(256) void k_remap(Dmda m, int b0, int b1, int b2, i
 }
 
 // ------------------------------------------------------------------ operator
-template <typename TX, bool DROP>
-__global__ __launch_bounds__(256) void k_apply64(Dims d, const double* __restrict__ g,
+template <typename TX, bool PAIRS>
+__global__ __launch_bounds__(256) void k_apply64(Dims d, uint32_t slab, const double* __restrict__ g,
                                                  const uint32_t* __restrict__ code, const TX* __restrict__ x,
                                                  double* __restrict__ y) {
+  const uint32_t e = xcd_block().x * 256u + threadIdx.x;
+  int i, j, k;
+  if constexpr (PAIRS) {
+    if (!flat_pair(d, e, slab, i, j, k)) return;
+    double w[2];
+    apply_pair(d, pair_at(d, i, j, k), g, code, x, y, w);
+  } else {
+    if (flat_cell(d, e, i, j, k)) apply_cell(d, g, code, x, y, i, j, k);
+  }
+}
+
+// the assembled matrix of the reference: coefficients with |v| <= 1e-10 dropped
+// (poisson.c:1608); needs the coefficients one by one
+template <typename TX>
+__global__ __launch_bounds__(256) void k_apply64_drop(Dims d, const double* __restrict__ g,
+                                                      const uint32_t* __restrict__ code, const TX* __restrict__ x,
+                                                      double* __restrict__ y) {
   CELL_IJK(i, j, k);
   if (i >= d.nx || j >= d.ny) return;
   const size_t c = d.idx(i, j, k);
   const uint32_t cd = code[c];
   Nbr nb;
   neighbours(d, i, j, k, nb);
-  double acc = 0.;
-  if constexpr (DROP) {
-    // the assembled matrix of the reference: coefficients with |v| <= 1e-10 dropped
-    // (poisson.c:1608); needs the coefficients one by one
-    double vol[19];
-    build_row(g, d.n(), cd, c, nb.s[WP], nb.s[SP], nb.s[BP], vol);
+  double vol[19], acc = 0.;
+  build_row(g, d.n(), cd, c, nb.s[WP], nb.s[SP], nb.s[BP], vol);
 #pragma unroll
-    for (int s = 0; s < 19; s++) {
-      double v = vol[s];
-      if (s != CP && !(fabs(v) > 1.e-10)) v = 0.;
-      if (v != 0.) acc += v * (double)x[nb.s[s]];
-    }
-  } else {
-    double xv[19], dg;
-    load_x(nb, x, xv);
-    flux_row(g, d.n(), cd, c, nb.s[WP], nb.s[SP], nb.s[BP], xv, acc, dg);
+  for (int s = 0; s < 19; s++) {
+    double v = vol[s];
+    if (s != CP && !(fabs(v) > 1.e-10)) v = 0.;
+    if (v != 0.) acc += v * (double)x[nb.s[s]];
   }
   y[c] = (cd & ROW_BIT) ? acc : 0.;
 }
 
-template <typename TX>
-__global__ __launch_bounds__(256) void k_residual64(Dims d, const double* __restrict__ g,
+// r = b - A x and per-block sums of r . r, bound like A x alone (k_apply64) by L1 with one
+// cell per thread and near HBM's rate with two (A x: 192x96x128 41.5 -> 33.3 us,
+// 131x77x93 26.0 -> 17.4, 512x256x256 888 -> 642).
+template <typename TX, bool PAIRS>
+__global__ __launch_bounds__(256) void k_residual64(Dims d, uint32_t slab, const double* __restrict__ g,
                                                     const uint32_t* __restrict__ code, const double* __restrict__ b,
                                                     const TX* __restrict__ x, double* __restrict__ r,
                                                     double* __restrict__ partial) {
   __shared__ double lds[4];
-  CELL_IJK(i, j, k);
-  double rr = 0.;
-  if (i < d.nx && j < d.ny) rr = residual_cell(d, g, code, b, x, r, i, j, k);
+  double rr = residual_at<PAIRS>(d, slab, xcd_block().x * 256u + threadIdx.x, g, code, b, x, r);
   rr = block_sum(rr, lds);
-  if (threadIdx.x == 0 && threadIdx.y == 0) partial[blin()] = rr;
+  if (threadIdx.x == 0) partial[blockIdx.x] = rr;
 }
 
 __global__ __launch_bounds__(256) void k_apply_dmda(Dmda m, Dims d, const double* __restrict__ g,
@@ -491,22 +504,18 @@ __global__ __launch_bounds__(256) void k_copy16(size_t n2, const double2* __rest
   if (t < n2) b[t] = a[t];
 }
 
-// w = A z (flux form) and per-wave partial sums of w.V_l (l < nv) and w.w (four
-// per 64x4 block); the first Krylov reduction of classical Gram-Schmidt fused
-// into the operator pass.
-template <typename TZ>
-__global__ __launch_bounds__(256) void k_apply_dots(Dims d, const double* __restrict__ g,
-                                                    const uint32_t* __restrict__ code, const TZ* __restrict__ z,
-                                                    double* __restrict__ w, const double* __restrict__ V, size_t ldv,
-                                                    int nv, double* __restrict__ partial) {
-  CELL_IJK(i, j, k);
-  const size_t nblk = (size_t)gridDim.x * gridDim.y * gridDim.z, b = blin();
-  const bool in = i < d.nx && j < d.ny;
-  const size_t c = in ? d.idx(i, j, k) : 0;
-  double v8[8];
-  wave_dots_prefetch(in, c, V, ldv, nv, v8);
-  const double wv = in ? apply_cell(d, g, code, z, w, i, j, k) : 0.;
-  wave_dots(in, c, wv, V, ldv, nv, v8, partial, 4 * nblk, 4 * b + threadIdx.y);
+// w = A z (flux form) and per-wave partial sums of w.V_l (l < nv) and w.w (four per block):
+// the first Krylov reduction of classical Gram-Schmidt fused into the operator pass.  With
+// two cells per thread it streams near HBM's rate.  With four vectors, one cell per thread
+// -> two: z in FP32 at 192x96x128 53.0 -> 46.0 us (6.0 TB/s), 131x77x93 25.1 -> 19.2,
+// 512x256x256 910 -> 826; z in FP64 at 192x96x128 69.3 -> 52.7, 64x64x64 8.5 -> 6.7.
+template <typename TZ, bool PAIRS>
+__global__ __launch_bounds__(256, 3) void k_apply_dots(Dims d, uint32_t slab, const double* __restrict__ g,
+                                                       const uint32_t* __restrict__ code, const TZ* __restrict__ z,
+                                                       double* __restrict__ w, const double* __restrict__ V,
+                                                       size_t ldv, int nv, double* __restrict__ partial) {
+  apply_dots<PAIRS>(d, slab, xcd_block().x * 256u + threadIdx.x, g, code, z, w, V, ldv, nv, partial,
+                    4 * (size_t)gridDim.x, 4 * (size_t)blockIdx.x + (threadIdx.x >> 6));
 }
 
 // CGS2 second pass, fused: w1 = w - sum_l h_l V_l (in place) and per-block
@@ -646,8 +655,11 @@ void launch_classify_nvert(hipStream_t s, Dmda m, const int bc[6], double* nv, u
 
 template <typename TX>
 void launch_apply64(hipStream_t s, Dims d, const double* g, const uint32_t* code, const TX* x, double* y, bool drop) {
-  if (drop) k_apply64<TX, true><<<cell_grid(d), kBlk, 0, s>>>(d, g, code, x, y);
-  else k_apply64<TX, false><<<cell_grid(d), kBlk, 0, s>>>(d, g, code, x, y);
+  const bool pairs = takes_pairs(d.n());
+  const unsigned nb = walk_blocks(d, pairs);
+  if (drop) k_apply64_drop<TX><<<cell_grid(d), kBlk, 0, s>>>(d, g, code, x, y);
+  else if (pairs) k_apply64<TX, true><<<nb, 256, 0, s>>>(d, pair_slab(d), g, code, x, y);
+  else k_apply64<TX, false><<<nb, 256, 0, s>>>(d, 0, g, code, x, y);
   HIPCHECK(hipGetLastError());
 }
 template void launch_apply64<double>(hipStream_t, Dims, const double*, const uint32_t*, const double*, double*, bool);
@@ -656,9 +668,11 @@ template void launch_apply64<float>(hipStream_t, Dims, const double*, const uint
 template <typename TX>
 void launch_residual64(hipStream_t s, Dims d, const double* g, const uint32_t* code, const double* b, const TX* x,
                        double* r, double* partial, int* nblk) {
-  const dim3 gr = cell_grid(d);
-  *nblk = (int)(gr.x * gr.y * gr.z);
-  k_residual64<TX><<<gr, kBlk, 0, s>>>(d, g, code, b, x, r, partial);
+  const bool pairs = takes_pairs(d.n());
+  const unsigned nb = walk_blocks(d, pairs);
+  *nblk = (int)nb;
+  if (pairs) k_residual64<TX, true><<<nb, 256, 0, s>>>(d, pair_slab(d), g, code, b, x, r, partial);
+  else k_residual64<TX, false><<<nb, 256, 0, s>>>(d, 0, g, code, b, x, r, partial);
   HIPCHECK(hipGetLastError());
 }
 template void launch_residual64<double>(hipStream_t, Dims, const double*, const uint32_t*, const double*,
@@ -876,9 +890,11 @@ void launch_fillf(hipStream_t s, size_t n, float* a, float v) {
 template <typename TZ>
 void launch_apply_dots(hipStream_t s, Dims d, const double* g, const uint32_t* code, const TZ* z, double* w,
                        const double* V, size_t ldv, int nv, double* partial, int* nblk) {
-  const dim3 gr = cell_grid(d);
-  *nblk = (int)(4 * gr.x * gr.y * gr.z);  // one partial per wave
-  k_apply_dots<TZ><<<gr, kBlk, 0, s>>>(d, g, code, z, w, V, ldv, nv, partial);
+  const bool pairs = takes_pairs(d.n());
+  const unsigned nb = walk_blocks(d, pairs);
+  *nblk = (int)(4 * nb);  // one partial per wave
+  if (pairs) k_apply_dots<TZ, true><<<nb, 256, 0, s>>>(d, pair_slab(d), g, code, z, w, V, ldv, nv, partial);
+  else k_apply_dots<TZ, false><<<nb, 256, 0, s>>>(d, 0, g, code, z, w, V, ldv, nv, partial);
   HIPCHECK(hipGetLastError());
 }
 template void launch_apply_dots<float>(hipStream_t, Dims, const double*, const uint32_t*, const float*, double*,

@@ -4,6 +4,7 @@
 #pragma once
 
 #include "pp_common.hpp"
+#include "pp_pair_dev.hpp"
 #include "pp_stencil.hpp"
 
 namespace pp {
@@ -68,38 +69,52 @@ __device__ __forceinline__ double wave_sum_to63(double v) {
   return v;
 }
 
-// V_l[c] for l < min(nv, 8), loaded before the value they multiply is computed so
-// the loads overlap that computation
-__device__ __forceinline__ void wave_dots_prefetch(bool in, size_t c, const double* __restrict__ V, size_t ldv,
-                                                   int nv, double (&v8)[8]) {
+// V_l on the N cells from c for l < min(nv, DOTS_AHEAD), loaded before the values they
+// multiply are computed so the loads overlap that computation
+constexpr int DOTS_AHEAD = 4;
+template <int N>
+__device__ __forceinline__ void wave_dots_prefetch(bool in, uint32_t c, const double* __restrict__ V, size_t ldv,
+                                                   int nv, double (&va)[DOTS_AHEAD][N]) {
 #pragma unroll
-  for (int q = 0; q < 8; q++) v8[q] = (in && q < nv) ? V[(size_t)q * ldv + c] : 0.;
+  for (int q = 0; q < DOTS_AHEAD; q++) {
+#pragma unroll
+    for (int m = 0; m < N; m++) va[q][m] = 0.;
+    if (in && q < nv) {
+      if constexpr (N == 2) ld_pair(V + (size_t)q * ldv, c, va[q]);
+      else va[q][0] = ld_at(V + (size_t)q * ldv, c);
+    }
+  }
 }
 
-// Per-wave sums of a * V_l[c] for l < nv and of a * a (slot nv), written by the
-// wave's last lane to partial[l * nw + wv] (nw waves in the launch, wv this
-// wave's index).  v8 holds V_l[c] for l < 8 (wave_dots_prefetch); the rest are
-// loaded eight at a time.  Every lane of the wave must call it (cells outside the
-// grid pass in = false); nv < 64.
-__device__ inline void wave_dots(bool in, size_t c, double a, const double* __restrict__ V, size_t ldv, int nv,
-                                 const double (&v8)[8], double* __restrict__ partial, size_t nw, size_t wv) {
+// Per-wave sums of a . V_l over each thread's N cells for l < nv and of a . a (slot nv),
+// written by the wave's last lane to partial[l * nw + wv] (nw waves in the launch, wv this
+// wave's index).  c is the first cell; a is 0 where a cell is another thread's.  va holds
+// the first DOTS_AHEAD vectors (wave_dots_prefetch); the rest are loaded as many at a time.
+// Every lane of the wave must call it (cells outside the grid pass in = false); nv < 64.
+template <int N>
+__device__ inline void wave_dots(bool in, uint32_t c, const double (&a)[N], const double* __restrict__ V, size_t ldv,
+                                 int nv, double (&va)[DOTS_AHEAD][N], double* __restrict__ partial, size_t nw,
+                                 size_t wv) {
   const int lane = (threadIdx.x + blockDim.x * (threadIdx.y + blockDim.y * threadIdx.z)) & 63;
-  for (int l0 = 0; l0 <= nv; l0 += 8) {
-    double p[8];
+  double own = 0.;
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-      const int l = l0 + q;
-      double v = 0.;
-      if (in && l < nv) v = a * (l0 == 0 ? v8[q] : V[(size_t)l * ldv + c]);
-      else if (in && l == nv) v = a * a;
-      p[q] = v;
+  for (int m = 0; m < N; m++) own += a[m] * a[m];
+  own = wave_sum_to63(in ? own : 0.);
+  if (lane == 63) partial[(size_t)nv * nw + wv] = own;
+  for (int l0 = 0; l0 < nv; l0 += DOTS_AHEAD) {
+    if (l0 > 0) wave_dots_prefetch(in, c, V + (size_t)l0 * ldv, ldv, nv - l0, va);
+    double p[DOTS_AHEAD];
+#pragma unroll
+    for (int q = 0; q < DOTS_AHEAD; q++) {
+      p[q] = 0.;
+#pragma unroll
+      for (int m = 0; m < N; m++) p[q] += a[m] * va[q][m];
+      p[q] = wave_sum_to63(in ? p[q] : 0.);
     }
-#pragma unroll
-    for (int q = 0; q < 8; q++) p[q] = wave_sum_to63(p[q]);
     if (lane == 63) {
 #pragma unroll
-      for (int q = 0; q < 8; q++)
-        if (l0 + q <= nv) partial[(size_t)(l0 + q) * nw + wv] = p[q];
+      for (int q = 0; q < DOTS_AHEAD; q++)
+        if (l0 + q < nv) partial[(size_t)(l0 + q) * nw + wv] = p[q];
     }
   }
 }
@@ -177,7 +192,23 @@ __host__ __device__ inline double conv_scale(double a2) {
   return ldexp(1.0, -(int)floor(0.5 * e));
 }
 
-// w[c] = (A z)[c] in flux form on a row cell, 0 elsewhere; returns w[c]
+// w = A z in flux form on the pair's row cells, 0 elsewhere; wv: w, 0 on a first cell that
+// is another thread's
+template <typename TZ>
+__device__ __forceinline__ void apply_pair(const Dims& d, const PairAt& at, const double* __restrict__ g,
+                                           const uint32_t* __restrict__ code, const TZ* __restrict__ z,
+                                           double* __restrict__ w, double (&wv)[2]) {
+  uint32_t cd[2];
+  PairX<TZ> xs;
+  double ax[2], dg[2];
+  pair_apply(at, g, d.n(), code, z, cd, xs, ax, dg);
+  const double w0 = (cd[0] & ROW_BIT) ? ax[0] : 0.;
+  wv[1] = (cd[1] & ROW_BIT) ? ax[1] : 0.;
+  wv[0] = at.both ? w0 : 0.;
+  st_pair(w, at.c, at.both, w0, wv[1]);
+}
+
+// the same on one cell
 template <typename TZ>
 __device__ __forceinline__ double apply_cell(const Dims& d, const double* __restrict__ g,
                                              const uint32_t* __restrict__ code, const TZ* __restrict__ z,
@@ -192,6 +223,32 @@ __device__ __forceinline__ double apply_cell(const Dims& d, const double* __rest
   const double wv = (cd & ROW_BIT) ? ax : 0.;
   w[c] = wv;
   return wv;
+}
+
+// w = A z on the cells of thread e (pairs: a flat walk of pairs, else of cells) and the
+// wave's partial sums of w.V_l (l < nv) and w.w; e is past the last on idle threads.
+template <bool PAIRS, typename TZ>
+__device__ __forceinline__ void apply_dots(const Dims& d, uint32_t slab, uint32_t e, const double* __restrict__ g,
+                                           const uint32_t* __restrict__ code, const TZ* __restrict__ z,
+                                           double* __restrict__ w, const double* __restrict__ V, size_t ldv, int nv,
+                                           double* __restrict__ partial, size_t nw, size_t wave) {
+  int i = 0, j = 0, k = 0;
+  if constexpr (PAIRS) {
+    const bool in = flat_pair(d, e, slab, i, j, k);
+    double va[DOTS_AHEAD][2], wv[2] = {0., 0.};
+    PairAt at{};
+    if (in) at = pair_at(d, i, j, k);
+    wave_dots_prefetch(in, at.c, V, ldv, nv, va);
+    if (in) apply_pair(d, at, g, code, z, w, wv);
+    wave_dots(in, at.c, wv, V, ldv, nv, va, partial, nw, wave);
+  } else {
+    const bool in = flat_cell(d, e, i, j, k);
+    const uint32_t c = in ? (uint32_t)d.idx(i, j, k) : 0u;
+    double va[DOTS_AHEAD][1], wv[1] = {0.};
+    wave_dots_prefetch(in, c, V, ldv, nv, va);
+    if (in) wv[0] = apply_cell(d, g, code, z, w, i, j, k);
+    wave_dots(in, c, wv, V, ldv, nv, va, partial, nw, wave);
+  }
 }
 
 // w1 = w - sum_l h_l V_l at element t (in place); returns w1

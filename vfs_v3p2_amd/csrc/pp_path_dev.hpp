@@ -6,6 +6,7 @@
 #pragma once
 
 #include "pp_kernels.hpp"
+#include "pp_pair_dev.hpp"
 #include "pp_stencil.hpp"
 
 namespace pp {
@@ -118,11 +119,28 @@ __device__ __forceinline__ void ibflux_correct_face(const IbFace& F, double* __r
 }
 
 // ----------------------------------------------------------- FP64 true residual
-// r[c] = b[c] - (A x)[c] on row cells, 0 elsewhere; returns r[c]^2
+// r = b - A x on the pair's row cells, 0 elsewhere; returns r . r over the cells that are
+// this thread's
 template <typename TX>
-__device__ inline double residual_cell(const Dims& d, const double* __restrict__ g, const uint32_t* __restrict__ code,
-                                       const double* __restrict__ b, const TX* __restrict__ x, double* __restrict__ r,
-                                       int i, int j, int k) {
+__device__ __forceinline__ double residual_pair(const Dims& d, const PairAt& at, const double* __restrict__ g,
+                                                const uint32_t* __restrict__ code, const double* __restrict__ b,
+                                                const TX* __restrict__ x, double* __restrict__ r) {
+  uint32_t cd[2];
+  PairX<TX> xs;
+  double bv[2], ax[2], dg[2];
+  ld_pair(b, at.c, bv);
+  pair_apply(at, g, d.n(), code, x, cd, xs, ax, dg);
+  const double r0 = (cd[0] & ROW_BIT) ? bv[0] - ax[0] : 0., r1 = (cd[1] & ROW_BIT) ? bv[1] - ax[1] : 0.;
+  st_pair(r, at.c, at.both, r0, r1);
+  return (at.both ? r0 * r0 : 0.) + r1 * r1;
+}
+
+// the same on one cell
+template <typename TX>
+__device__ __forceinline__ double residual_cell(const Dims& d, const double* __restrict__ g,
+                                                const uint32_t* __restrict__ code, const double* __restrict__ b,
+                                                const TX* __restrict__ x, double* __restrict__ r, int i, int j,
+                                                int k) {
   const size_t c = d.idx(i, j, k);
   const uint32_t cd = code[c];
   Nbr nb;
@@ -133,6 +151,15 @@ __device__ inline double residual_cell(const Dims& d, const double* __restrict__
   const double res = (cd & ROW_BIT) ? b[c] - ax : 0.;
   r[c] = res;
   return res * res;
+}
+// the residual on the cells of thread e (pairs: a flat walk of pairs, else of cells)
+template <bool PAIRS, typename TX>
+__device__ __forceinline__ double residual_at(const Dims& d, uint32_t slab, uint32_t e, const double* __restrict__ g,
+                                              const uint32_t* __restrict__ code, const double* __restrict__ b,
+                                              const TX* __restrict__ x, double* __restrict__ r) {
+  int i, j, k;
+  if constexpr (PAIRS) return flat_pair(d, e, slab, i, j, k) ? residual_pair(d, pair_at(d, i, j, k), g, code, b, x, r) : 0.;
+  else return flat_cell(d, e, i, j, k) ? residual_cell(d, g, code, b, x, r, i, j, k) : 0.;
 }
 
 // |aj r| on Divergence-counted cells: with r = b - A phi this is the max |aj div u|
