@@ -235,3 +235,35 @@ def test_tile_shapes_give_identical_results(E, torch_cuda):
             np.testing.assert_array_equal(a, c)
             np.testing.assert_array_equal(b, d)
             assert ia == ic
+
+
+@pytest.mark.parametrize("dims", [(65, 34, 33), (129, 33, 17), (64, 32, 31), (67, 30, 32), (131, 30, 18), (33, 32, 64)])
+@pytest.mark.parametrize("precision", [1, 0])
+def test_pair_and_cell_kernels_agree(E, torch_cuda, dims, precision):
+    """A case alone and in a batch of one take different kernels at these sizes (FP64
+    smoothing and restriction by pairs from 65536 cells on, against cells in the batch;
+    restriction by pairs in the batch from 64 columns or 65536 cells on): odd and even
+    rows and planes, with a sphere.  Both run the same V-cycle, so two iterations leave the
+    same Phi up to rounding amplified by the solve: relative L2 1e-4 eps32 ~ 1e-6 for FP32
+    V-cycles (a rounding of the smoothed correction, relative to it) and 1e-11 in FP64; a
+    wrong row or coarse cell changes it by far more."""
+    torch = torch_cuda
+    nx, ny, nz = dims
+    cs = [(cases.hill_case(nx, ny, nz, h=0.2, beta=1.2, sphere=(0.6, 0.9, 0.0, 0.25), seed=4), None)]
+    c = cs[0][0]
+    print(f"pairs against cells: {c.name}, precision {precision}", flush=True)
+    fluid = c.fields["nvert"] < 0.1
+    fluid[0], fluid[-1], fluid[:, 0], fluid[:, -1], fluid[:, :, 0], fluid[:, :, -1] = (False,) * 6
+    kw = dict(precision=precision, rtol=1e-14, div_tol=0.0, smoother=1, max_iters=2, fused=0)
+    h, = handles(E, cs, **kw)
+    u, phi, p, ucat = fields(torch, cs)
+    h.project(u[0], phi[0], p[0], ucat[0], c.dt, c.st, c.coeff)
+    h.close()
+    hs = handles(E, cs, **kw)
+    B = E.Batch(hs)
+    u2, phi2, p2, ucat2 = fields(torch, cs)
+    B.project(u2, phi2, p2, ucat2, [c.dt], [c.st], [c.coeff])
+    B.close()
+    hs[0].close()
+    a, b = phi[0].cpu().numpy(), phi2[0].cpu().numpy()
+    assert relL2(b, a, fluid) <= (1e-6 if precision == 1 else 1e-11)

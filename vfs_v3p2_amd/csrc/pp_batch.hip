@@ -140,7 +140,6 @@ struct RestrictItem {
   const T* r;  // general: the fine residual f - A x (written by a kb_resid launch before)
   int cmask;
   int slot;
-  uint32_t tx, ty;  // blk: 64x2x2 fine tiles; general: 64x4x1 coarse tiles
 };
 
 template <typename T>
@@ -273,18 +272,16 @@ __global__ __launch_bounds__(64 * Y::W) void kb_line_step(const SmoothItem<T>* _
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void kb_restrict_blk(const RestrictItem<T>* __restrict__ items,
+__global__ __launch_bounds__(256) void kb_restrict_pairs(const RestrictItem<T>* __restrict__ items,
                                                        const uint32_t* __restrict__ start, int nitems, uint32_t total,
                                                        const SlotDev* __restrict__ sd) {
-  __shared__ T lds[2][2][32];
+  __shared__ T lds[2][2][64];
   FOR_TILES(total, t) {
     const uint32_t tw_ = start[nitems + t];
     const int q = (int)(tw_ >> 16);
     const RestrictItem<T>& I = items[q];
     if (!sd[tw_ & 0xffffu].y) continue;
-    const uint32_t lt = t - start[q];
-    resid_restrict_blk(I.F, I.f, I.x, I.dc, I.clsc, I.fc, (int)(lt % I.tx), (int)((lt / I.tx) % I.ty),
-                       (int)(lt / (I.tx * I.ty)), I.cmask == 5, lds);
+    resid_restrict_pairs(I.F, I.f, I.x, I.dc, I.clsc, I.fc, t - start[q], I.cmask == 5, lds);
   }
 }
 
@@ -983,6 +980,8 @@ struct BatchCore {
         std::vector<RestrictItem<T>> rb, rg;
         std::vector<SmoothItem<T>> rr;  // fine residuals of the general restriction
         std::vector<uint32_t> nb, ng;
+        size_t cells = 0;
+        for (int q : sm) cells += slots[q].mg->lev[d].d.n();
         for (int q : sm) {
           auto& L = slots[q].mg->lev[d];
           auto& C = slots[q].mg->lev[d + 1];
@@ -995,17 +994,14 @@ struct BatchCore {
           it.fc = C.f;
           it.cmask = (C.d.nx != L.d.nx ? 1 : 0) | (C.d.ny != L.d.ny ? 2 : 0) | (C.d.nz != L.d.nz ? 4 : 0);
           it.slot = q;
-          if ((it.cmask == 7 || it.cmask == 5) && L.d.nx >= 64) {  // narrower levels: flat cells fill the lanes better
-            it.tx = (uint32_t)(L.d.nx + 63) / 64;
-            it.ty = (uint32_t)(L.d.ny + 1) / 2;
+          if ((it.cmask == 7 || it.cmask == 5) && (L.d.nx >= 64 || takes_pairs(cells))) {
+            const uint32_t tile = restrict_tile(it.cmask == 5);
             rb.push_back(it);
-            nb.push_back(it.tx * it.ty * (uint32_t)((L.d.nz + 1) / 2));
+            nb.push_back((uint32_t)((C.d.n() + tile - 1) / tile));
           } else {
             // the fine residual goes to the level's direction buffer, which no step
             // reads between the end of the pre-smoothing and the first
             // post-smoothing step (a new Chebyshev sequence, c1 = 0)
-            it.tx = (uint32_t)(C.d.nx + 63) / 64;
-            it.ty = (uint32_t)(C.d.ny + 3) / 4;
             it.r = L.dv;
             rg.push_back(it);
             ng.push_back(cell_tiles(C.d));
@@ -1237,8 +1233,7 @@ struct BatchCore {
         });
         break;
       case K_RBLK:
-        kb_restrict_blk<T><<<W, dim3(64, 2, 2), 0, s>>>(static_cast<const RestrictItem<T>*>(L.items), L.start,
-                                                        L.nitems, L.total, sd);
+        kb_restrict_pairs<T><<<W, 256, 0, s>>>(static_cast<const RestrictItem<T>*>(L.items), L.start, L.nitems, L.total, sd);
         break;
       case K_RGEN:
         kb_restrict_gen<T><<<W, dim3(64, 4, 1), 0, s>>>(static_cast<const RestrictItem<T>*>(L.items), L.start,

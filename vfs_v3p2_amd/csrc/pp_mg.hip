@@ -38,6 +38,17 @@ __global__ __launch_bounds__(256) void k_smooth_point(LevelView<T> L, const T* _
   smooth_point_cell<T, MODE>(L, f, dinv, x_old, x_prev, x_new, dv, c1, c2, c0, i, j, k, fd);
 }
 
+// k_smooth_point with two cells per thread (see pp_pair_dev.hpp)
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void k_smooth_pairs(LevelView<T> L, uint32_t slab, const T* __restrict__ f,
+                                                      const T* __restrict__ dinv, const T* __restrict__ x_old,
+                                                      T* x_prev, T* x_new, T c1, T c2, T c0,
+                                                      const T* __restrict__ fd) {
+  int p, j, k;
+  if (!flat_pair(L.d, xcd_block().x * 256u + threadIdx.x, slab, p, j, k)) return;
+  smooth_point_pair<T, MODE>(L, f, dinv, x_old, x_prev, x_new, c1, c2, c0, pair_at(L.d, p, j, k), fd);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_line_rows(LevelView<T> L, T* __restrict__ lfac) {
   CELL_IJK(i, j, k);
@@ -132,6 +143,15 @@ __global__ __launch_bounds__(256) void k_resid_restrict_blk(LevelView<T> F, cons
   __shared__ T lds[2][2][32];
   const uint3 xb = xcd_block();
   resid_restrict_blk(F, f, x, dc, clsc, fc, (int)xb.x, (int)xb.y, (int)xb.z, keep_y != 0, lds);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_resid_restrict_pairs(LevelView<T> F, const T* __restrict__ f,
+                                                              const T* __restrict__ x, Dims dc,
+                                                              const uint8_t* __restrict__ clsc, T* __restrict__ fc,
+                                                              int keep_y) {
+  __shared__ T lds[2][2][64];
+  resid_restrict_pairs(F, f, x, dc, clsc, fc, xcd_block().x, keep_y != 0, lds);
 }
 
 template <typename T>
@@ -620,6 +640,21 @@ void launch_smooth(hipStream_t s, LevelView<T> L, const T* lfac, int mode, const
                                                                  c2);
     }
   } else {
+    if constexpr (sizeof(T) == 8) {
+      // two cells per thread from FP64 coefficients; FP32 levels read FP16 ones and 4-byte
+      // values, which L1 serves at its full rate one cell per thread, and lose more to the
+      // registers of two (192x96x128: FP32 15.9 -> 20.0 us, FP64 48.7 -> 39.0)
+      if (takes_pairs(L.d.n()) && (mode == SM_NEXT || mode == SM_FIRST2)) {
+        const unsigned nb = (pair_count(L.d) + 255) / 256;
+        const uint32_t slab = pair_slab(L.d);
+        if (mode == SM_NEXT)
+          k_smooth_pairs<T, SM_NEXT><<<nb, 256, 0, s>>>(L, slab, f, dinv, x_old, x_prev, x_new, c1, c2, c0, fd);
+        else
+          k_smooth_pairs<T, SM_FIRST2><<<nb, 256, 0, s>>>(L, slab, f, dinv, x_old, x_prev, x_new, c1, c2, c0, fd);
+        HIPCHECK(hipGetLastError());
+        return;
+      }
+    }
     switch (mode) {
       case SM_ZERO:
         k_smooth_point<T, SM_ZERO><<<cell_grid(L.d), kBlk, 0, s>>>(L, f, dinv, x_old, x_prev, x_new, dv, c1, c2, c0, fd);
@@ -678,6 +713,15 @@ template <typename T>
 void launch_resid_restrict(hipStream_t s, LevelView<T> F, const T* f, const T* x, Dims dc, const uint8_t* cls_c,
                            T* fc) {
   const int cm = (dc.nx != F.d.nx ? 1 : 0) | (dc.ny != F.d.ny ? 2 : 0) | (dc.nz != F.d.nz ? 4 : 0);
+  if constexpr (sizeof(T) == 8) {
+    if ((cm == 7 || cm == 5) && takes_pairs(F.d.n())) {
+      const uint32_t tile = restrict_tile(cm == 5);
+      k_resid_restrict_pairs<T><<<(unsigned)((dc.n() + tile - 1) / tile), 256, 0, s>>>(F, f, x, dc, cls_c, fc,
+                                                                                      cm == 5 ? 1 : 0);
+      HIPCHECK(hipGetLastError());
+      return;
+    }
+  }
   if (cm == 7 || cm == 5) {  // 2x2x2 children, or 2x1x2 (i and k coarsened, j kept)
     const dim3 gr((F.d.nx + 63) / 64, (F.d.ny + 1) / 2, (F.d.nz + 1) / 2);
     k_resid_restrict_blk<T><<<gr, dim3(64, 2, 2), 0, s>>>(F, f, x, dc, cls_c, fc, cm == 5 ? 1 : 0);

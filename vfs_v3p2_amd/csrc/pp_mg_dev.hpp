@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "pp_kernels.hpp"
+#include "pp_pair_dev.hpp"
 #include "pp_stencil.hpp"
 
 namespace pp {
@@ -152,6 +153,93 @@ __device__ __forceinline__ void smooth_point_cell(const LevelView<T>& L, const T
     }
     smooth_point_body<T, MODE>(L, L.g, false, f, dinv, x_old, x_prev, x_new, dv, c1, c2, c0, i, j, k, fd);
   }
+}
+
+// (A x) and the diagonal on a pair from x already loaded, with the class bytes picking the
+// row form (see flux_by_class); row: which of the two cells have one
+template <typename T, typename TG>
+__device__ __forceinline__ void pair_by_class(const LevelView<T>& L, const TG* __restrict__ g, bool scaled,
+                                              const PairAt& at, PairX<T>& xs, T (&ax)[2], T (&dg)[2],
+                                              bool (&row)[2]) {
+  uint8_t cl[2];
+  PairG<TG> gs;
+  ld_pair(L.cls, at.c, cl);
+  pair_load_g(at, g, L.d.n(), gs);
+  pair_share_x(at, xs);
+  pair_share_g(at, gs);
+  row[0] = row[1] = true;
+  if (__all((cl[0] & CLS_INTERIOR) && (cl[1] & CLS_INTERIOR))) {
+    const uint32_t cd[2] = {CODE_INTERIOR, CODE_INTERIOR};
+    pair_flux<X_CENTRAL>(gs, xs, cd, ax, dg);
+  } else {
+    uint32_t cd[2];
+    ld_pair(L.code, at.c, cd);
+    pair_flux<-1>(gs, xs, cd, ax, dg);
+    row[0] = (cd[0] & ROW_BIT) != 0;
+    row[1] = (cd[1] & ROW_BIT) != 0;
+  }
+  if (scaled) {
+#pragma unroll
+    for (int m = 0; m < 2; m++) ax[m] *= L.gs, dg[m] *= L.gs;
+  }
+}
+
+// smooth_point_body on a pair of cells (SM_NEXT, SM_FIRST2)
+template <typename T, int MODE, typename TG>
+__device__ __forceinline__ void smooth_pair_body(const LevelView<T>& L, const TG* __restrict__ g, bool scaled,
+                                                 const T* __restrict__ f, const T* __restrict__ dinv,
+                                                 const T* __restrict__ x_old, T* x_prev, T* x_new, T c1, T c2, T c0,
+                                                 const PairAt& at, const T* __restrict__ fd) {
+  T fc[2], xp[2] = {T(0), T(0)}, xn[2];
+  PairX<T> xs;
+  ld_pair(f, at.c, fc);
+  if constexpr (MODE == SM_NEXT) {
+    if (c1 != T(0)) ld_pair((const T*)x_prev, at.c, xp);
+    pair_load_x(at, x_old, xs);
+  } else {
+    pair_load_x(at, fd ? fd : f, xs);
+    if (fd) {
+#pragma unroll
+      for (int s = 0; s < 9; s++) xs.v[s][0] *= c0, xs.v[s][1] *= c0;
+#pragma unroll
+      for (int s = 0; s < 5; s++) xs.l[s] *= c0, xs.r[s] *= c0;
+    } else {
+      PairX<T> ds;
+      pair_load_x(at, dinv, ds);
+#pragma unroll
+      for (int s = 0; s < 9; s++)
+        xs.v[s][0] = c0 * (xs.v[s][0] * ds.v[s][0]), xs.v[s][1] = c0 * (xs.v[s][1] * ds.v[s][1]);
+#pragma unroll
+      for (int s = 0; s < 5; s++) xs.l[s] = c0 * (xs.l[s] * ds.l[s]), xs.r[s] = c0 * (xs.r[s] * ds.r[s]);
+    }
+  }
+  T ax[2], dg[2];
+  bool row[2];
+  pair_by_class(L, g, scaled, at, xs, ax, dg, row);
+#pragma unroll
+  for (int m = 0; m < 2; m++) {
+    const bool live = row[m] && dg[m] != T(0);
+    const T z = live ? (fc[m] - ax[m]) / (live ? dg[m] : T(1)) : T(0);
+    const T xc = xs.v[0][m];
+    const T dold = MODE == SM_FIRST2 ? xc : (c1 == T(0) ? T(0) : xc - xp[m]);
+    xn[m] = row[m] ? xc + (c1 * dold + c2 * z) : T(0);
+  }
+  if constexpr (MODE == SM_FIRST2)
+    st_pair(x_prev, at.c, at.both, row[0] ? xs.v[0][0] : T(0), row[1] ? xs.v[0][1] : T(0));
+  st_pair(x_new, at.c, at.both, xn[0], xn[1]);
+}
+template <typename T, int MODE>
+__device__ __forceinline__ void smooth_point_pair(const LevelView<T>& L, const T* __restrict__ f,
+                                                  const T* __restrict__ dinv, const T* __restrict__ x_old,
+                                                  T* x_prev, T* x_new, T c1, T c2, T c0, const PairAt& at,
+                                                  const T* __restrict__ fd) {
+  if constexpr (std::is_same<T, float>::value) {
+    if (L.gh) {
+      smooth_pair_body<T, MODE>(L, L.gh, true, f, dinv, x_old, x_prev, x_new, c1, c2, c0, at, fd);
+      return;
+    }
+  }
+  smooth_pair_body<T, MODE>(L, L.g, false, f, dinv, x_old, x_prev, x_new, c1, c2, c0, at, fd);
 }
 
 // Thomas factors of the y-line tridiagonal part of A on the line (i, k), from the
@@ -415,6 +503,57 @@ __device__ __forceinline__ void resid_restrict_blk(const LevelView<T>& F, const 
       const T v = (lds[0][0][tx] + lds[0][1][tx]) + (lds[1][0][tx] + lds[1][1][tx]);
       fc[C] = (clsc[C] & CLS_NONFLUID) ? T(0) : v;
     }
+  }
+  __syncthreads();  // the LDS tile is reused by the block's next tile
+}
+
+// f - A x on a pair's rows, 0 elsewhere and on a first cell that is another thread's
+template <typename T>
+__device__ __forceinline__ T resid_pair_sum(const LevelView<T>& L, const T* __restrict__ f, const T* __restrict__ x,
+                                            const PairAt& at) {
+  T fc[2], ax[2], dg[2];
+  bool row[2];
+  PairX<T> xs;
+  ld_pair(f, at.c, fc);
+  pair_load_x(at, x, xs);
+  if constexpr (std::is_same<T, float>::value) {
+    if (L.gh) pair_by_class(L, L.gh, true, at, xs, ax, dg, row);
+    else pair_by_class(L, L.g, false, at, xs, ax, dg, row);
+  } else {
+    pair_by_class(L, L.g, false, at, xs, ax, dg, row);
+  }
+  const T r0 = (at.both && row[0]) ? fc[0] - ax[0] : T(0), r1 = row[1] ? fc[1] - ax[1] : T(0);
+  return r0 + r1;
+}
+
+// Coarse cells of one block of resid_restrict_pairs
+HDI uint32_t restrict_tile(bool keep_y) { return keep_y ? 128u : 64u; }
+
+// Residual + restriction as in resid_restrict_blk (the same sums in the same order) for
+// tile `tile` of the level's coarse cells in flat order, so levels of any width fill every
+// lane: a thread takes the two children adjacent in i, the block's four waves the two or
+// four rows of them (j kept: two rows, 128 coarse cells).  Every thread of the 256-thread
+// block must call it.
+template <typename T>
+__device__ __forceinline__ void resid_restrict_pairs(const LevelView<T>& F, const T* __restrict__ f,
+                                                     const T* __restrict__ x, const Dims& dc,
+                                                     const uint8_t* __restrict__ clsc, T* __restrict__ fc,
+                                                     uint32_t tile, bool keep_y, T (*lds)[2][64]) {
+  const int lane = threadIdx.x & 63, lo = (threadIdx.x >> 6) & 1, hi = threadIdx.x >> 7;
+  const uint32_t E = keep_y ? tile * 128u + 64u * lo + lane : tile * 64u + lane;
+  int ic, jc, kc;
+  const bool in = flat_cell(dc, E, ic, jc, kc);
+  T r = T(0);
+  if (in) {
+    const int j = keep_y ? jc : 2 * jc + lo, k = 2 * kc + hi;
+    if (j < F.d.ny && k < F.d.nz) r = resid_pair_sum(F, f, x, pair_at(F.d, ic, j, k));
+  }
+  lds[hi][lo][lane] = r;
+  __syncthreads();
+  if (in && hi == 0 && (keep_y || lo == 0)) {
+    const T v = keep_y ? lds[0][lo][lane] + lds[1][lo][lane]
+                       : (lds[0][0][lane] + lds[0][1][lane]) + (lds[1][0][lane] + lds[1][1][lane]);
+    fc[E] = (clsc[E] & CLS_NONFLUID) ? T(0) : v;
   }
   __syncthreads();  // the LDS tile is reused by the block's next tile
 }
