@@ -310,8 +310,9 @@ __global__ __launch_bounds__(256) void kb_prolong(const ProlongItem<T>* __restri
     const ProlongItem<T>& I = items[q];
     if (!sd[tw_ & 0xffffu].y) continue;
     int i, j, k;
-    if (!shaped_cell(shape, I.F.d, t - start[q], i, j, k)) continue;
-    prolong_add_cell(I.F, I.dc, I.clsc, I.cmask, I.xc, I.xf, i, j, k);
+    if (!shaped_cell(shape, prolong_dims(I.F.d, I.dc, I.cmask), t - start[q], i, j, k)) continue;
+    if (I.cmask & 1) prolong_add_pair(I.F, I.dc, I.clsc, I.cmask, I.xc, I.xf, i, j, k);
+    else prolong_add_cell(I.F, I.dc, I.clsc, I.cmask, I.xc, I.xf, i, j, k);
   }
 }
 
@@ -1142,7 +1143,7 @@ struct BatchCore {
   // walks); starts with the flat walk, the tuner may pick another shape.
   static Dims cells_of(const SmoothItem<T>& I) { return I.L.d; }
   static Dims cells_of(const RestrictItem<T>& I) { return I.dc; }
-  static Dims cells_of(const ProlongItem<T>& I) { return I.F.d; }
+  static Dims cells_of(const ProlongItem<T>& I) { return prolong_dims(I.F.d, I.dc, I.cmask); }
   template <typename Item>
   void add_launch_cells(int kind, int mode, const std::vector<Item>& items) {
     if (items.empty()) return;

