@@ -1000,7 +1000,7 @@ struct BatchCore {
             rb.push_back(it);
             nb.push_back((uint32_t)((C.d.n() + tile - 1) / tile));
           } else {
-            // the fine residual goes to the level's direction buffer, which no step
+            // the fine residual goes to the level's power-iteration buffer, which no step
             // reads between the end of the pre-smoothing and the first
             // post-smoothing step (a new Chebyshev sequence, c1 = 0)
             it.r = L.dv;

@@ -1278,8 +1278,9 @@ int vfs_pp_mg_nvert_restrict_device(const vfs_grid* g, const double* nvf, double
 // Algorithmic bytes per cell of one finest-level Chebyshev sweep: a point sweep
 // reads x, f, the coefficients and the mask and writes x (FP32 level with FP16
 // coefficients 31, FP64 97); a y-line step whose lines fit the segmented layout
-// reads x, f, coefficients, mask, the three Thomas factors and the direction and
-// writes the direction and x (51 / 137); on longer lines the residual goes through
+// counts x, f, coefficients, mask, three Thomas factors, the previous iterate twice and
+// the x it writes (51 / 137; the FP32 step reads its 24 bytes of row records in place of
+// coefficients and factors); on longer lines the residual goes through
 // memory (x, f, g, mask -> r, then r, factors, x -> x: 55 / 145).
 static double sweep_bytes_per_cell(const vfs_pp_handle* h) {
   const bool f32 = h->opts.precision == 1;
@@ -1365,7 +1366,7 @@ int vfs_pp_time_kernel(vfs_pp_handle* h, int kernel, int reps, double* ms, doubl
   *ms = (double)tms / reps;
   // Algorithmic bytes per launch: each distinct array once per cell, halos from
   // cache, a 1-byte mask per cell.  (The engine's kernels move somewhat more:
-  // a 4-byte branch-code word instead of the mask, and the Chebyshev direction.)
+  // a 4-byte branch-code word instead of the mask, and the previous Chebyshev iterate.)
   const double N = (double)n;
   switch (kernel) {
     case 0: *bytes = N * (8 + 72 + 1 + 8); break;  // phi, g11..g33, mask -> y           = 89

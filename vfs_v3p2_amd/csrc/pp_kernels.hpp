@@ -239,9 +239,9 @@ inline int line_layout(int ny, size_t lines) {
 // with c1 = 0, c2 = 1 from f = 0 that stores D^-1 (f - A x) in dv (power iteration)
 enum { SM_NEXT = 0, SM_ZERO = 1, SM_FIRST2 = 2, SM_POWER = 3 };
 
-// Point levels keep the previous iterate in x_prev (x_new may be the same buffer:
-// each cell reads its own x_prev before writing x_new); y-line levels keep the
-// Chebyshev direction in dv and ignore x_prev.  fd (optional, point levels in
+// One Chebyshev step in three-term form with the previous iterate in x_prev (x_new may be
+// the same buffer: each cell reads its own x_prev before writing x_new; on y-line levels
+// x_prev may be null for zero).  dv: SM_POWER's result.  fd (optional, point levels in
 // SM_FIRST2): f * dinv as stored by the writer of f.
 template <typename T>
 void launch_smooth(hipStream_t s, LevelView<T> L, const T* lfac, int mode, const T* f, const T* dinv,
