@@ -427,7 +427,9 @@ __device__ __forceinline__ double tile_sum_wide(const double* __restrict__ pv, u
 // with c_l = red[8 + l] red[RED_NUINV2 + l] (w.U_l / |U_l|^2), the next V-cycle's
 // input f0 = (T)(w' s) with s = conv_scale(|w|^2 = red[8 + j + 1]), and per-wave
 // partial sums of |w'|^2 at partial[4 t + wave] (no LDS and no barrier per tile).
-// The same per-element arithmetic as k_axpy_norm.
+// 512 elements per tile, two per thread: a persistent worker's chain of dependent reads per
+// tile (list, item, slot, scalars) and its waits per vector held it at 4 TB/s (64 cases:
+// 405 -> 300 us; the single-case kernel, which has no such chain, gained nothing).
 template <typename T>
 __global__ __launch_bounds__(256) void kb_axpy_norm(const VecItem<T>* __restrict__ items,
                                                     const uint32_t* __restrict__ start, int nitems, uint32_t total,
@@ -439,17 +441,12 @@ __global__ __launch_bounds__(256) void kb_axpy_norm(const VecItem<T>* __restrict
     const SlotDev st = sd[tw_ & 0xffffu];
     if (!st.y) continue;
     const int nv = st.x + 1;
-    const size_t e = (size_t)(t - start[q]) * 256 + threadIdx.x;
-    double acc[1] = {0.};
-    if (e < I.n) {
-      double* w = I.V + (size_t)nv * I.n;
-      double v = w[e];
-      for (int l = 0; l < nv; l++) v -= (I.red[8 + l] * I.red[RED_NUINV2 + l]) * I.V[(size_t)l * I.n + e];
-      w[e] = v;
-      I.f0[e] = (T)(v * conv_scale(I.red[8 + nv]));
-      acc[0] = v * v;
-    }
-    const double ws = wave_sum_to63(acc[0]);
+    const uint32_t e = (t - start[q]) * 256u + threadIdx.x, n = (uint32_t)I.n;
+    const double v2 = 2 * (size_t)e < I.n
+                          ? axpy_norm_pair<T>(e, n, I.V + (size_t)nv * I.n, I.V, I.n, nv, I.red + 8,
+                                              I.red + RED_NUINV2, conv_scale(I.red[8 + nv]), I.f0)
+                          : 0.;
+    const double ws = wave_sum_to63(v2);
     if ((threadIdx.x & 63) == 63) partial[4 * (size_t)t + (threadIdx.x >> 6)] = ws;
   }
 }
@@ -1083,6 +1080,7 @@ struct BatchCore {
       size_t cells = 0;
       for (int q : mem) cells += slots[q].h->d.n();
       const bool pairs = takes_pairs(cells);
+      const size_t per = lazy ? 512 : 256;  // elements per tile of the basis passes
       for (int q : mem) {
         vfs_pp_handle* h = slots[q].h;
         const size_t n = h->d.n();
@@ -1106,7 +1104,7 @@ struct BatchCore {
         v.f0 = static_cast<T*>(slots[q].mg->f0());
         v.n = n;
         v.slot = q;
-        const uint32_t nv = (uint32_t)((n + 255) / 256);
+        const uint32_t nv = (uint32_t)((n + per - 1) / per);
         fv.push_back(FinItem{h->red, h->hpin_dev, tv, tv + nv, q});
         tv += nv;
         vi.push_back(v);

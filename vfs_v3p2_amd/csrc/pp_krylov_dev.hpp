@@ -251,6 +251,35 @@ __device__ __forceinline__ void apply_dots(const Dims& d, uint32_t slab, uint32_
   }
 }
 
+// The lazily normalised Gram-Schmidt update on the elements 2t and 2t + 1 (of an odd n the
+// last thread's pair overlaps the one before and stores its second element only):
+// w' = w - sum_l (dots_l nuinv2_l) V_l in place, f = (T)(w' sc).  Four vectors' pairs are
+// loaded at a time, so a thread waits for memory once per four vectors instead of once per
+// vector and element.  Returns |w'|^2 over the elements stored.
+template <typename T>
+__device__ __forceinline__ double axpy_norm_pair(uint32_t t, uint32_t n, double* __restrict__ w,
+                                                 const double* __restrict__ V, size_t ldv, int nv,
+                                                 const double* __restrict__ dots, const double* __restrict__ nuinv2,
+                                                 double sc, T* __restrict__ f) {
+  const uint32_t e = min(2 * t, n - 2);
+  const bool both = e == 2 * t;
+  double va[DOTS_AHEAD][2], v[2];
+  ld_pair((const double*)w, e, v);
+  for (int l0 = 0; l0 < nv; l0 += DOTS_AHEAD) {
+    wave_dots_prefetch(true, e, V + (size_t)l0 * ldv, ldv, nv - l0, va);
+#pragma unroll
+    for (int q = 0; q < DOTS_AHEAD; q++)
+      if (l0 + q < nv) {
+        const double c = dots[l0 + q] * nuinv2[l0 + q];
+        v[0] -= c * va[q][0];
+        v[1] -= c * va[q][1];
+      }
+  }
+  st_pair(w, e, both, v[0], v[1]);
+  st_pair(f, e, both, (T)(v[0] * sc), (T)(v[1] * sc));
+  return (both ? v[0] * v[0] : 0.) + v[1] * v[1];
+}
+
 // w1 = w - sum_l h_l V_l at element t (in place); returns w1
 __device__ __forceinline__ double gs_sub(double* __restrict__ w, const double* __restrict__ V, size_t ldv, int nv,
                                          const double* __restrict__ h, size_t t) {
