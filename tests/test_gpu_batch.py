@@ -237,12 +237,49 @@ def test_tile_shapes_give_identical_results(E, torch_cuda):
             assert ia == ic
 
 
+@pytest.mark.parametrize("smoother", [1, 2])
+@pytest.mark.parametrize("precision", [1, 0])
+def test_results_do_not_depend_on_the_members_beside(E, torch_cuda, precision, smoother):
+    """A member's Phi, Ucont, P and Ucat are the same bits in a batch of one and beside
+    members that take the batch across every bound of the kernel choices: 65536 cells, and
+    4096, 8192 and 16384 y-lines.  Members: narrow levels below 65536 cells, one above;
+    lines of up to 64, 128, 192, 224 and 256 rows with few lines each, one with 5184 lines
+    of 136 rows and one with 16384 lines.  Six iterations, whether converged or not."""
+    torch = torch_cuda
+    dims = [(24, 20, 28), (40, 40, 40), (20, 100, 24), (20, 140, 24), (20, 200, 24), (20, 240, 24), (72, 136, 72),
+            (128, 66, 128)]
+    cs = []
+    for q, (nx, ny, nz) in enumerate(dims):
+        sphere = (0.6, 0.9, 0.0, 0.3) if q % 2 else None
+        cs.append((cases.hill_case(nx, ny, nz, h=0.2, beta=1.5, sphere=sphere, seed=20 + q), None))
+    print(f"members alone and together, precision {precision}, smoother {smoother}", flush=True)
+    kw = dict(precision=precision, smoother=smoother, rtol=1e-14, div_tol=0.0, max_iters=6)
+
+    def run(sub):
+        hs = handles(E, sub, **kw)
+        B = E.Batch(hs)
+        u, phi, p, ucat = fields(torch, sub)
+        sts = B.project(u, phi, p, ucat, [c.dt for c, _ in sub], [c.st for c, _ in sub], [c.coeff for c, _ in sub])
+        B.close()
+        for h in hs:
+            h.close()
+        return [([x.cpu().numpy() for x in row], st.iterations) for row, st in zip(zip(u, phi, p, ucat), sts)]
+
+    together = run(cs)
+    for q, one in enumerate(cs):
+        (alone, it), = run([one])
+        print(f"  {one[0].name}", flush=True)
+        assert it == together[q][1] == 6
+        for a, b in zip(alone, together[q][0]):
+            np.testing.assert_array_equal(a, b)
+
+
 @pytest.mark.parametrize("dims", [(65, 34, 33), (129, 33, 17), (64, 32, 31), (67, 30, 32), (131, 30, 18), (33, 32, 64)])
 @pytest.mark.parametrize("precision", [1, 0])
 def test_pair_and_cell_kernels_agree(E, torch_cuda, dims, precision):
     """A case alone and in a batch of one take different kernels at these sizes (FP64
-    smoothing and restriction by pairs from 65536 cells on, against cells in the batch;
-    restriction by pairs in the batch from 64 columns or 65536 cells on): odd and even
+    smoothing and restriction by pairs from 65536 cells on, against smoothing by cells and
+    restriction by pairs in the batch): odd and even
     rows and planes, with a sphere.  Both run the same V-cycle, so two iterations leave the
     same Phi up to rounding amplified by the solve: relative L2 1e-4 eps32 ~ 1e-6 for FP32
     V-cycles (a rounding of the smoothed correction, relative to it) and 1e-11 in FP64; a

@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256) void kb_dense(const DenseItem<T>* __restrict__
 
 // w = A z_j (FP64 flux form) into V_{j+1}; per-wave partial sums of w.V_l (l <= j)
 // and w.w at partial[l * 4 total + 4 t + wave]
-template <typename T, bool PAIRS>
+template <typename T>
 __global__ __launch_bounds__(256, 3) void kb_apply_dots(const ApplyItem<T>* __restrict__ items,
                                                      const uint32_t* __restrict__ start, int nitems, uint32_t total,
                                                      const SlotDev* __restrict__ sd, double* __restrict__ partial) {
@@ -345,9 +345,9 @@ __global__ __launch_bounds__(256, 3) void kb_apply_dots(const ApplyItem<T>* __re
     const ApplyItem<T>& I = items[q];
     const SlotDev st = sd[tw_ & 0xffffu];
     if (!st.y) continue;
-    apply_dots<PAIRS>(I.d, pair_slab(I.d), (t - start[q]) * 256u + threadIdx.x, I.g, I.code,
-                      I.Z + (size_t)st.x * I.n, I.V + (size_t)(st.x + 1) * I.n, I.V, I.n, st.x + 1, partial,
-                      4 * (size_t)total, 4 * (size_t)t + (threadIdx.x >> 6));
+    apply_dots<true>(I.d, pair_slab(I.d), (t - start[q]) * 256u + threadIdx.x, I.g, I.code,
+                     I.Z + (size_t)st.x * I.n, I.V + (size_t)(st.x + 1) * I.n, I.V, I.n, st.x + 1, partial,
+                     4 * (size_t)total, 4 * (size_t)t + (threadIdx.x >> 6));
   }
 }
 
@@ -927,7 +927,7 @@ struct BatchCore {
         it.tx = (uint32_t)(L.d.nx + 63) / 64;
         it.ty = 0;
         if (seg_lines(L.d)) {
-          const int lay = line_layout<T>(L.d.ny, lines);
+          const int lay = line_layout<T>(L.d.ny, (size_t)L.d.nx * L.d.nz, lines);
           smode = mode;
           sg[lay].push_back(it);
           nsg[lay].push_back(seg_line_tiles(L.d, lay));
@@ -978,8 +978,6 @@ struct BatchCore {
         std::vector<RestrictItem<T>> rb, rg;
         std::vector<SmoothItem<T>> rr;  // fine residuals of the general restriction
         std::vector<uint32_t> nb, ng;
-        size_t cells = 0;
-        for (int q : sm) cells += slots[q].mg->lev[d].d.n();
         for (int q : sm) {
           auto& L = slots[q].mg->lev[d];
           auto& C = slots[q].mg->lev[d + 1];
@@ -992,7 +990,7 @@ struct BatchCore {
           it.fc = C.f;
           it.cmask = (C.d.nx != L.d.nx ? 1 : 0) | (C.d.ny != L.d.ny ? 2 : 0) | (C.d.nz != L.d.nz ? 4 : 0);
           it.slot = q;
-          if ((it.cmask == 7 || it.cmask == 5) && (L.d.nx >= 64 || takes_pairs(cells))) {
+          if (it.cmask == 7 || it.cmask == 5) {  // by pairs whatever the size (as the operator)
             const uint32_t tile = restrict_tile(it.cmask == 5);
             rb.push_back(it);
             nb.push_back((uint32_t)((C.d.n() + tile - 1) / tile));
@@ -1077,9 +1075,6 @@ struct BatchCore {
       std::vector<FinItem> fa, fv;
       uint32_t ta = 0, tv = 0;
       int mmax = 1;
-      size_t cells = 0;
-      for (int q : mem) cells += slots[q].h->d.n();
-      const bool pairs = takes_pairs(cells);
       const size_t per = lazy ? 512 : 256;  // elements per tile of the basis passes
       for (int q : mem) {
         vfs_pp_handle* h = slots[q].h;
@@ -1092,7 +1087,9 @@ struct BatchCore {
         a.V = h->V;
         a.n = n;
         a.slot = q;
-        const uint32_t na = pairs ? (pair_count(h->d) + 255) / 256 : cell_tiles(h->d);
+        // by pairs whatever the size: a rule on the cells of the whole plan would make a
+        // case's sums depend on what runs beside it
+        const uint32_t na = (pair_count(h->d) + 255) / 256;
         fa.push_back(FinItem{h->red, h->hpin_dev, ta, ta + na, q});
         ta += na;
         ai.push_back(a);
@@ -1121,7 +1118,7 @@ struct BatchCore {
       for (size_t q = 0; q < vi.size(); q++) { sv[q] = acc; acc += vn[q]; }
       auto pa = upload(ai, sa, ta);
       auto pv = upload(vi, sv, tv);
-      apply = Launch{K_APPLY, pairs ? 1 : 0, pa.first, pa.second, (int)ai.size(), ta, 2048};
+      apply = Launch{K_APPLY, 0, pa.first, pa.second, (int)ai.size(), ta, 2048};
       axd = Launch{K_AXD, 0, pv.first, pv.second, (int)vi.size(), tv, 2048};
       axs = Launch{K_AXS, 0, pv.first, pv.second, (int)vi.size(), tv, 2048};
       axn = Launch{K_AXN, 0, pv.first, pv.second, (int)vi.size(), tv, 2048};
@@ -1246,12 +1243,8 @@ struct BatchCore {
         kb_dense<T><<<W, 256, 0, s>>>(static_cast<const DenseItem<T>*>(L.items), L.start, L.nitems, L.total, sd);
         break;
       case K_APPLY:
-        if (L.mode)
-          kb_apply_dots<T, true><<<W, 256, 0, s>>>(static_cast<const ApplyItem<T>*>(L.items), L.start, L.nitems,
-                                                   L.total, sd, partial);
-        else
-          kb_apply_dots<T, false><<<W, 256, 0, s>>>(static_cast<const ApplyItem<T>*>(L.items), L.start, L.nitems,
-                                                    L.total, sd, partial);
+        kb_apply_dots<T><<<W, 256, 0, s>>>(static_cast<const ApplyItem<T>*>(L.items), L.start, L.nitems, L.total, sd,
+                                           partial);
         break;
       case K_AXD:
         kb_axpy_dots<T><<<W, 256, 0, s>>>(static_cast<const VecItem<T>*>(L.items), L.start, L.nitems, L.total, sd,

@@ -208,10 +208,11 @@ template <typename T>
 HD inline bool line_seg_fits(const Dims& d) {
   return d.ny <= 256;
 }
-// Block layout of the segmented step for lines of ny rows, `lines` of them in the
-// launch (all members of a batched one): an index into line_layouts<T>.  Few lines take
-// narrow blocks of few waves, so that every CU gets some and a block's barriers cost
-// little; many lines take wide ones, whose 256-byte accesses stream from HBM better.
+// Block layout of the segmented step for lines of ny rows of a level of `own` lines, in a
+// launch of `all` lines (a batched launch holds its members' levels): an index into
+// with_line_layout's layouts.  Few lines take narrow blocks of few waves, so that every CU
+// gets some and a block's barriers cost little; many lines take wide ones, whose 256-byte
+// accesses stream from HBM better.
 // The bounds are where the measured step times cross, in us (narrow / middle / wide):
 // FP32 64x64x64 6.4 / 7.2 / 9.5, 256x64x256 37.4 / 37.3 / 41.2, 64x100x64 - / 9.0 / 12.2,
 // 100x110x100 - / 20.5 / 15.8, 64x200x32 10.9 / 18.3 / 20.4, 128x256x64 21.7 / 20.5 / 27.3,
@@ -220,19 +221,23 @@ HD inline bool line_seg_fits(const Dims& d) {
 // x waves x lanes): 256x150x200 332 / 278 / 285 / 306, 100x200x100 69.3 / - / 82.7 / 80.0,
 // 256x200x128 247 / - / 232 / 237, 128x256x64 65.9 / - / 51.6 / 49.0, 512x256x256 1141 / - /
 // 1119 / 1098.
+// The number of segments per line sets how the line's sweeps round, so it follows from the
+// level's own lines alone; the launch's lines pick among layouts of that many segments (16,
+// or 32 in FP32 layout 4 and FP64 layouts 1 and 4), which give the same bits.  A batched
+// member's results therefore do not depend on the members beside it.
 constexpr int LINE_LAYOUTS = 7;
 template <typename T>
-inline int line_layout(int ny, size_t lines) {
+inline int line_layout(int ny, size_t own, size_t all) {
   if (sizeof(T) == 4) {
-    if (ny <= 64) return lines < 8192 ? 0 : 1;
-    if (ny <= 128) return lines < 8192 ? 2 : 3;
-    return lines < 4096 ? 4 : lines < 16384 ? 5 : 6;
+    if (ny <= 64) return all < 8192 ? 0 : 1;
+    if (ny <= 128) return all < 8192 ? 2 : 3;
+    return own < 4096 ? 4 : all < 16384 ? 5 : 6;
   }
   if (ny <= 64) return 0;
-  if (ny <= 128) return lines < 8192 ? 1 : 2;
-  if (ny <= 192) return lines < 8192 ? 1 : 3;
-  if (ny <= 224) return lines < 16384 ? 1 : 4;
-  return lines < 8192 ? 1 : 5;
+  if (ny <= 128) return own < 8192 ? 1 : 2;
+  if (ny <= 192) return own < 8192 ? 1 : 3;
+  if (ny <= 224) return all < 16384 ? 1 : 4;
+  return own < 8192 ? 1 : 5;
 }
 
 // Chebyshev smoothing launch modes (see smooth_point_cell); SM_POWER is one step

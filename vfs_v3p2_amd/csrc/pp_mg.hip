@@ -614,9 +614,10 @@ inline unsigned nb1(size_t n) { return (unsigned)((n + 255) / 256); }
 template <typename T>
 static void launch_line_step(hipStream_t s, const LevelView<T>& L, int mode, const T* f, const T* lfac,
                              const T* x_old, const T* x_prev, T* x_new, T c1, T c2) {
-  with_line_layout<T>(line_layout<T>(L.d.ny, (size_t)L.d.nx * L.d.nz), [&](auto lay) {
+  const size_t lines = (size_t)L.d.nx * L.d.nz;
+  with_line_layout<T>(line_layout<T>(L.d.ny, lines, lines), [&](auto lay) {
     using Y = decltype(lay);
-    const dim3 gr((unsigned)(((size_t)L.d.nx * L.d.nz + Y::LANES - 1) / Y::LANES)), bl(64, Y::W);
+    const dim3 gr((unsigned)((lines + Y::LANES - 1) / Y::LANES)), bl(64, Y::W);
     if (mode == LS_ZERO)
       k_line_step<T, Y, LS_ZERO><<<gr, bl, 0, s>>>(L, f, lfac, x_old, x_prev, x_new, c1, c2);
     else if (mode == LS_POWER)
