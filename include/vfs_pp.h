@@ -188,8 +188,13 @@ int vfs_pp_formfunction2_device(const vfs_grid *grid, const double *icsi, const 
  * place; dp is Pressure_Gradient's output (vfs_pp_pressure_gradient_device).
  * The inflow/outflow boundary (InflowFlux, FormBCS) and the IB velocity
  * interpolation (ibm_interpolation_advanced) are the caller's: Contra2Cart
- * leaves the Ucat of IB-adjacent cells as passed.  Allocates 10 vector-field
- * scratch arrays per call. */
+ * leaves the Ucat of IB-adjacent cells as passed.  Works on 10 vector-field
+ * scratch arrays (240 bytes per DMDA point).
+ *
+ * Scratch of the momentum calls on a handle (this one, vfs_pp_momentum_residual_device,
+ * vfs_pp_implicit_momentum_device): the handle keeps its scratch for the next call while
+ * all handles of the process together keep at most 8 GiB, and frees it when the call
+ * returns otherwise.  vfs_pp_destroy frees it, and so does joining a batch. */
 int vfs_pp_runge_kutta_device(vfs_pp_handle *h, const double *icsi, const double *ieta, const double *izet,
                               const double *jcsi, const double *jeta, const double *jzet,
                               const double *kcsi, const double *keta, const double *kzet,
@@ -245,7 +250,9 @@ typedef struct {
  * differ while the solution meets the same test.  Afterwards the solution's wall
  * faces are zeroed as Implicit_MatrixFree does (implicitsolver.c:408-415) and
  * ucat receives its Contra2Cart.  VFS_PP_ENOCONV if the tolerance was not met
- * (ucont then holds the last iterate); stats may be NULL. */
+ * (ucont then holds the last iterate); stats may be NULL.  Works on 43 vector-field
+ * scratch arrays, 45 with slip walls or immersed == 3 (about 1050 bytes per DMDA point;
+ * kept as vfs_pp_runge_kutta_device says). */
 int vfs_pp_implicit_momentum_device(vfs_pp_handle *h, const double *icsi, const double *ieta,
                                     const double *izet, const double *jcsi, const double *jeta,
                                     const double *jzet, const double *kcsi, const double *keta,

@@ -385,3 +385,54 @@ def test_implicit_form_refusals(E, torch_cuda):
         E.momentum_residual(h, met, z, u, u, 100.0, 0.01, coeff=1.5)
     assert ei.value.code == E.VFS_PP_EINVAL
     h.close()
+
+
+def test_momentum_work_vectors_are_bounded_and_given_back(E, torch_cuda):
+    """Five handles that take an implicit step each (about 2.3 GB of work vectors apiece)
+    keep at most 8 GiB of them between calls: the ones beyond it give theirs back and step
+    to the same bits.  Joining a batch and destroying a handle free them."""
+    torch = torch_cuda
+    c = cases.channel_case(128, 126, 128, beta=1.5, seed=3)
+    met = {k: dev(torch, c.fields[k]) for k in METRICS}
+    uo = dev(torch, np.ascontiguousarray(c.fields["ucont"]))
+    zero, u, ucat = torch.zeros_like(uo), torch.zeros_like(uo), torch.zeros_like(uo)
+    first = torch.zeros_like(uo)
+
+    def step(h):
+        u.copy_(uo)
+        st = E.Implicit_MatrixFree(h, met, zero, uo, u, ucat, 400.0, 1e-3, 1.0, rhs_o=zero, rtol=0.5, max_newton=2,
+                                   strict=False)
+        torch.cuda.synchronize()
+        return st.newton_iterations
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    gib = 1 << 30
+    hs = []
+    for _ in range(5):
+        h = E.Handle(E.make_grid(c.nx, c.ny, c.nz, c.per, c.bctype, 0), E.default_opts())
+        h.set_geometry(c.fields)
+        hs.append(h)
+    f0 = free()
+    assert step(hs[0]) >= 1
+    first.copy_(u)
+    assert f0 - free() > 2 * gib  # kept
+    for h in hs[1:] + hs[:2]:
+        step(h)
+        assert torch.equal(u, first)
+    print(f"five handles keep {(f0 - free()) / gib:.2f} GiB", flush=True)
+    assert f0 - free() <= 8 * gib + gib // 8
+    before = free()
+    B = E.Batch(hs[:1])
+    assert free() - before > gib
+    B.close()
+    for h in hs:
+        h.close()
+    h = E.Handle(E.make_grid(c.nx, c.ny, c.nz, c.per, c.bctype, 0), E.default_opts())
+    h.set_geometry(c.fields)
+    f1 = free()
+    step(h)
+    assert torch.equal(u, first) and f1 - free() > 2 * gib  # the bound is free again
+    h.close()

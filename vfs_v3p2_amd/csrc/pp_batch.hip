@@ -799,6 +799,7 @@ struct BatchCore {
     if (!mg) throw StatusError(VFS_PP_EINVAL, "batch members must share the multigrid precision");
     if (degree == 0) degree = mg->degree;
     if (mg->degree != degree) throw StatusError(VFS_PP_EINVAL, "batch members must share cheb_degree");
+    h->mom_free();  // no momentum step runs on a bound handle
     sl.h = h;
     sl.mg = mg;
     sl.own_stream = h->s;

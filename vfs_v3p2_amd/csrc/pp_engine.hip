@@ -921,6 +921,7 @@ int vfs_pp_destroy(vfs_pp_handle* h) {
   if (h->s) (void)hipStreamSynchronize(h->s);
   h->mg.reset();
   h->ar.release();
+  h->mom_free();
   if (h->hpin) (void)hipHostFree(h->hpin);
   if (h->ev) (void)hipEventDestroy(h->ev);
   if (h->s) (void)hipStreamDestroy(h->s);

@@ -5,6 +5,7 @@
 #pragma once
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <map>
@@ -371,6 +372,14 @@ struct MG : MGBase {
   }
 };
 
+// Momentum work vectors the process's handles keep between calls, in bytes, and their
+// bound: an explicit step's take 240 B per point and an implicit step's 1050, so without
+// one every handle of a large grid would hold on to a sizable part of the card (35 GB at
+// 512x256x256).  8 GiB is 3% of it and holds the vectors of an implicit step of 8 M points,
+// where allocating them anew costs the step about a fifth at any size.
+constexpr size_t MOM_KEEP = (size_t)8 << 30;
+inline std::atomic<size_t> mom_kept{0};
+
 }  // namespace pp
 
 struct vfs_pp_handle {
@@ -386,15 +395,33 @@ struct vfs_pp_handle {
   // device bytes the handle holds: grid-sized buffers, the geometry's, set-up scratch and
   // momentum work vectors
   size_t resident_bytes() const { return ar.total() + geo.total() + setup_tmp.total() + mom.total(); }
-  pp::Arena mom;  // momentum work vectors, from the first momentum step on (mom_buf)
-  std::vector<std::pair<double*, size_t>> mom_bufs;
-  // work vector q of the momentum steps, at least n doubles; kept by the handle, since
-  // allocating and freeing about 1 GB per call cost an implicit step of 1.2 M cells about 2 ms.  Only
-  // points the steps write are ever read, and a handle's grid never changes.
+  pp::Arena mom;  // momentum work vectors (mom_buf)
+  std::vector<double*> mom_bufs;
+  size_t mom_counted = 0;  // this handle's part of mom_kept
+  // work vector q of the momentum steps, n doubles.  Kept between the handle's calls where
+  // MOM_KEEP allows (mom_settle), since allocating and freeing about 1 GB per call cost an
+  // implicit step of 1.2 M cells about 2 ms.  Only points the steps write are ever read; q's
+  // size follows from the grid, which never changes.
   double* mom_buf(size_t q, size_t n) {
-    if (mom_bufs.size() <= q) mom_bufs.resize(q + 1, {nullptr, 0});
-    if (mom_bufs[q].second < n) mom_bufs[q] = {mom.alloc<double>(n), n};
-    return mom_bufs[q].first;
+    if (mom_bufs.size() <= q) mom_bufs.resize(q + 1, nullptr);
+    if (!mom_bufs[q]) mom_bufs[q] = mom.alloc<double>(n);
+    return mom_bufs[q];
+  }
+  // at the end of a momentum call: the work vectors stay with the handle if all handles'
+  // together stay within MOM_KEEP, else they are freed
+  void mom_settle() {
+    const size_t t = mom.total();
+    size_t kept = pp::mom_kept.load(), rest;
+    do rest = kept - mom_counted;
+    while (!pp::mom_kept.compare_exchange_weak(kept, rest + t <= pp::MOM_KEEP ? rest + t : rest));
+    mom_counted = rest + t <= pp::MOM_KEEP ? t : 0;
+    if (mom_counted != t) mom_free();
+  }
+  void mom_free() {
+    mom.release();
+    mom_bufs.clear();
+    pp::mom_kept -= mom_counted;
+    mom_counted = 0;
   }
   double* hstage = nullptr;   // device copies of vfs_pp_project's host arrays (8 M doubles, from ar)
   int batch_refs = 0;         // batches / server slots the handle is bound to (0 or 1)

@@ -757,6 +757,12 @@ struct ImplicitMomentum {
   }
 };
 
+// the handle's work vectors, kept or given back when a momentum call ends either way
+struct MomScope {
+  vfs_pp_handle* h;
+  ~MomScope() { h->mom_settle(); }
+};
+
 // checks shared by the implicit entry points
 void implicit_setup(vfs_pp_handle* h, const double* const met[15], const double* dp, const double* uo,
                     const double* urm1, double ren, double dt, double coeff, ImplicitMomentum& P) {
@@ -834,6 +840,7 @@ int vfs_pp_runge_kutta_device(vfs_pp_handle* h, const double* icsi, const double
   vfs_grid gr = h->grid;
   gr.immersed = h->immersed_ref;
   const MomIn in = make_in(&gr, met, h->nvert);
+  MomScope scope{h};
   double* ws = h->mom_buf(0, 8 * M3);
   double* pu = h->mom_buf(1, M3);
   double* rhs = h->mom_buf(2, M3);
@@ -877,6 +884,7 @@ int vfs_pp_momentum_residual_device(vfs_pp_handle* h, const double* icsi, const 
   const double* met[15] = {icsi, ieta, izet, jcsi, jeta, jzet, kcsi, keta, kzet, iaj, jaj, kaj, csi, eta, zet};
   for (auto p : met)
     if (!p) return VFS_PP_EINVAL;
+  MomScope scope{h};
   ImplicitMomentum P;
   implicit_setup(h, met, dp, ucont_o, ucont_rm1, ren, dt, coeff, P);
   P.rhs_o = rhs_o;
@@ -899,6 +907,7 @@ int vfs_pp_implicit_momentum_device(vfs_pp_handle* h, const double* icsi, const 
   const double* met[15] = {icsi, ieta, izet, jcsi, jeta, jzet, kcsi, keta, kzet, iaj, jaj, kaj, csi, eta, zet};
   for (auto p : met)
     if (!p) return VFS_PP_EINVAL;
+  MomScope scope{h};
   ImplicitMomentum P;
   implicit_setup(h, met, dp, ucont_o, ucont_rm1, ren, dt, coeff, P);
   P.rhs_o = rhs_o;
