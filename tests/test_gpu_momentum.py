@@ -214,12 +214,13 @@ def _uniform_flux(f, U):
     return u
 
 
-def test_implicit_step_of_a_uniform_flow(E, torch_cuda):
+@pytest.mark.parametrize("dims", [(10, 9, 11), (9, 7, 11)])  # the second with an odd number of points
+def test_implicit_step_of_a_uniform_flow(E, torch_cuda, dims):
     """A uniform flow on a periodic sheared grid has no Formfunction_2 part, so
     F(U) = -(U - Uo)/dt - dP is linear and its root is the uniform flux of
     Uo - dt dU: the Newton-Krylov solve lands on it."""
     torch = torch_cuda
-    c = _periodic_affine()
+    c = _periodic_affine(*dims)
     f = c.fields
     U0, Uo, dU = np.array([0.8, -0.4, 0.3]), np.array([0.7, -0.3, 0.2]), np.array([0.2, 0.1, -0.3])
     u0, uo, dp = _uniform_flux(f, U0), _uniform_flux(f, Uo), _uniform_flux(f, dU)
