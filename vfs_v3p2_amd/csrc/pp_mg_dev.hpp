@@ -184,12 +184,13 @@ __device__ __forceinline__ void pair_by_class(const LevelView<T>& L, const TG* _
   }
 }
 
-// smooth_point_body on a pair of cells (SM_NEXT, SM_FIRST2)
-template <typename T, int MODE, typename TG>
-__device__ __forceinline__ void smooth_pair_body(const LevelView<T>& L, const TG* __restrict__ g, bool scaled,
-                                                 const T* __restrict__ f, const T* __restrict__ dinv,
-                                                 const T* __restrict__ x_old, T* x_prev, T* x_new, T c1, T c2, T c0,
-                                                 const PairAt& at, const T* __restrict__ fd) {
+// smooth_point_cell on a pair of cells of an FP64 level (SM_NEXT, SM_FIRST2)
+template <typename T, int MODE>
+__device__ __forceinline__ void smooth_point_pair(const LevelView<T>& L, const T* __restrict__ f,
+                                                  const T* __restrict__ dinv, const T* __restrict__ x_old,
+                                                  T* x_prev, T* x_new, T c1, T c2, T c0, const PairAt& at,
+                                                  const T* __restrict__ fd) {
+  static_assert(std::is_same<T, double>::value, "FP32 levels take one cell per thread (launch_smooth)");
   T fc[2], xp[2] = {T(0), T(0)}, xn[2];
   PairX<T> xs;
   ld_pair(f, at.c, fc);
@@ -215,7 +216,7 @@ __device__ __forceinline__ void smooth_pair_body(const LevelView<T>& L, const TG
   }
   T ax[2], dg[2];
   bool row[2];
-  pair_by_class(L, g, scaled, at, xs, ax, dg, row);
+  pair_by_class(L, L.g, false, at, xs, ax, dg, row);
 #pragma unroll
   for (int m = 0; m < 2; m++) {
     const bool live = row[m] && dg[m] != T(0);
@@ -228,20 +229,6 @@ __device__ __forceinline__ void smooth_pair_body(const LevelView<T>& L, const TG
     st_pair(x_prev, at.c, at.both, row[0] ? xs.v[0][0] : T(0), row[1] ? xs.v[0][1] : T(0));
   st_pair(x_new, at.c, at.both, xn[0], xn[1]);
 }
-template <typename T, int MODE>
-__device__ __forceinline__ void smooth_point_pair(const LevelView<T>& L, const T* __restrict__ f,
-                                                  const T* __restrict__ dinv, const T* __restrict__ x_old,
-                                                  T* x_prev, T* x_new, T c1, T c2, T c0, const PairAt& at,
-                                                  const T* __restrict__ fd) {
-  if constexpr (std::is_same<T, float>::value) {
-    if (L.gh) {
-      smooth_pair_body<T, MODE>(L, L.gh, true, f, dinv, x_old, x_prev, x_new, c1, c2, c0, at, fd);
-      return;
-    }
-  }
-  smooth_pair_body<T, MODE>(L, L.g, false, f, dinv, x_old, x_prev, x_new, c1, c2, c0, at, fd);
-}
-
 // Thomas factors of the y-line tridiagonal part of A on the line (i, k), from the
 // rows' SP / CP / NP coefficients (cells without an unknown get the identity):
 // lfac = [a | cp | inv], each n long; den_j = b_j - a_j cp_{j-1}, inv_j = 1/den_j,
