@@ -566,8 +566,9 @@ int vfs_pp_server_status(vfs_pp_server *sv, int *queued, int *active, size_t *re
  * the finest level is smoothed by y-lines).  Writes the mean duration (ms) and
  * the algorithmic bytes of one launch: every distinct array once per cell, with
  * a 1-byte mask (apply 89, smoother 31 FP32 (FP16 coefficients) / 97 FP64, or
- * for a y-line finest level its fused residual + line step 51 / 137 (lines of
- * up to 256 rows) or separate residual + line solve 55 / 145, projection 129,
+ * for a y-line finest level its fused residual + line step 40 or 44 / 113 or 129
+ * (lines of up to 256 rows, by the block layout) or separate residual + line solve
+ * 59 / 153, both with the previous iterate, projection 129,
  * Contra2Cart 121, RHS 33 bytes per cell, Krylov pass z + 72 + 1 + 8 + 4 x 8 =
  * 117 (FP32 z) / 121, streaming floor 35 / 105; copy 16 bytes per element). */
 int vfs_pp_time_kernel(vfs_pp_handle *h, int kernel, int reps, double *ms_per_launch,

@@ -563,7 +563,7 @@ def test_kernel_timer_ids(E, torch_cuda):
     """vfs_pp_time_kernel: every id times its kernel and states its algorithmic
     bytes (point levels: sweep 31 B/cell in FP32, streaming floor 35); a y-line
     finest level has no point-sweep streaming floor (EINVAL) and prices its fused
-    residual + line step at 51 B/cell."""
+    residual + line step at 40 B/cell (records 24, x, previous x, f and the x it writes)."""
     c = get_case("hill_sphere")[0]
     h = handle_for(E, c, precision=1, smoother=1)
     n = c.nx * c.ny * c.nz
@@ -575,7 +575,7 @@ def test_kernel_timer_ids(E, torch_cuda):
     h.close()
     ch = cases.channel_case(16, 64, 12, beta=3.0, seed=2)
     h = handle_for(E, ch, precision=1, smoother=2)
-    assert h.time_kernel(1, 3)[1] == 51 * ch.nx * ch.ny * ch.nz
+    assert h.time_kernel(1, 3)[1] == 40 * ch.nx * ch.ny * ch.nz
     with pytest.raises(E.VfsPPError) as ei:
         h.time_kernel(8, 3)
     assert ei.value.code == E.VFS_PP_EINVAL

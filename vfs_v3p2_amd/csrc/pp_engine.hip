@@ -83,7 +83,7 @@ static std::vector<double> coarse_bordered(const CoarseRows& L, int* ncomp_out) 
   return B;
 }
 
-// The elimination of launch_gj_panel (partial pivoting on the first largest
+// The elimination of launch_gj_panel (partial pivoting, here on the first largest
 // |B[r][col]|) column by column on [B | I] on the host: it returns the top-left n x n
 // block of B^-1, column-major.
 static std::vector<double> coarse_inverse_host(std::vector<double> B, int N, int n) {
@@ -1278,17 +1278,17 @@ int vfs_pp_mg_nvert_restrict_device(const vfs_grid* g, const double* nvf, double
 
 // Algorithmic bytes per cell of one finest-level Chebyshev sweep: a point sweep
 // reads x, f, the coefficients and the mask and writes x (FP32 level with FP16
-// coefficients 31, FP64 97); a y-line step whose lines fit the segmented layout
-// counts x, f, coefficients, mask, three Thomas factors, the previous iterate twice and
-// the x it writes (51 / 137; the FP32 step reads its 24 bytes of row records in place of
-// coefficients and factors); on longer lines the residual goes through
-// memory (x, f, g, mask -> r, then r, factors, x -> x: 55 / 145).
+// coefficients 31, FP64 97); a segmented y-line step reads x, the previous iterate, f and
+// its coefficients (line_step_coef_bytes) and writes x (40 or 44 / 113 or 129); on longer
+// lines the residual goes through memory (x, f, g, mask -> r, then r, factors, x, the
+// previous iterate -> x: 59 / 153).
 static double sweep_bytes_per_cell(const vfs_pp_handle* h) {
   const bool f32 = h->opts.precision == 1;
-  if (!h->mg->line0()) return f32 ? (4 + 4 + 18 + 1 + 4) : (8 + 8 + 72 + 1 + 8);
+  const double t = f32 ? 4 : 8, g = f32 ? 18 : 72;
+  if (!h->mg->line0()) return t + t + g + 1 + t;
   const bool seg = f32 ? line_seg_fits<float>(h->d) : line_seg_fits<double>(h->d);
-  if (seg) return f32 ? (4 + 4 + 18 + 1 + 12 + 8 + 4) : (8 + 8 + 72 + 1 + 24 + 16 + 8);
-  return f32 ? (4 + 4 + 18 + 1 + 4) + (4 + 12 + 4 + 4) : (8 + 8 + 72 + 1 + 8) + (8 + 24 + 8 + 8);
+  if (seg) return 4 * t + (f32 ? line_step_coef_bytes<float>(h->d) : line_step_coef_bytes<double>(h->d));
+  return (t + t + g + 1 + t) + (t + 3 * t + t + t + t);
 }
 
 int vfs_pp_time_kernel(vfs_pp_handle* h, int kernel, int reps, double* ms, double* bytes) {

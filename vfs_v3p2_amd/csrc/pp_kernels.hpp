@@ -257,6 +257,10 @@ void launch_line_factors(hipStream_t s, LevelView<T> L, T* lfac);
 // Thomas factors
 void launch_line_pack(hipStream_t s, const LevelView<float>& L, const float* lfac, u32x2* pi, u32x2* pj,
                       u32x2* pk);
+// bytes per cell of the coefficients, class byte and Thomas factors that the segmented
+// y-line step on level d reads
+template <typename T>
+double line_step_coef_bytes(const Dims& d);
 // streaming floor of a point sweep: reads every array the sweep reads once per
 // cell (class byte, nine coefficient arrays, f, x, the previous iterate) and
 // writes one, with no stencil

@@ -160,7 +160,11 @@ struct LineLds {
 //   0 the residual (a and 1 / den are read after the walk, cp and x with them);
 //   1 the upward sweep's two values per row (cp and x are read after the walk);
 //   2 those, cp and x (nothing is read twice).
-// LM and KEEP are bounded by the 128 registers a wave may have with four waves per SIMD.
+// LM and KEEP are bounded by registers.  In FP32 every layout stays within the 128 that
+// leave four waves per SIMD (88 to 114 for a step from x, 94 to 120 batched).  In FP64
+// they do not all: 146, 131, 158 and 200 registers in layouts 0, 1, 3 and 5 (3, 3, 3 and 2
+// waves per SIMD), and the 1024-thread blocks of layouts 2 and 4 are held to 128 and spill
+// 4 and 2 (batched 8 and 12); they are still the faster ones where line_layout picks them.
 template <int LM_, int W_, int LANES_, int KEEP_>
 struct LineLayout {
   static constexpr int LM = LM_, W = W_, LANES = LANES_, S = W_ * 64 / LANES_, KEEP = KEEP_;

@@ -628,6 +628,19 @@ static void launch_line_step(hipStream_t s, const LevelView<T>& L, int mode, con
 }
 
 template <typename T>
+double line_step_coef_bytes(const Dims& d) {
+  int keep = 0;
+  const size_t lines = (size_t)d.nx * d.nz;
+  with_line_layout<T>(line_layout<T>(d.ny, lines, lines), [&](auto lay) { keep = decltype(lay)::KEEP; });
+  // FP32: the three records, and cp where it is read after the walk; FP64: coefficients,
+  // class byte and 1 / den, and a and cp where they are read after the walk
+  if (sizeof(T) == 4) return 24 + (keep < 2 ? 4 : 0) + (keep < 1 ? 4 : 0);
+  return 72 + 1 + 8 + (keep < 2 ? 8 : 0) + (keep < 1 ? 8 : 0);
+}
+template double line_step_coef_bytes<float>(const Dims&);
+template double line_step_coef_bytes<double>(const Dims&);
+
+template <typename T>
 void launch_smooth(hipStream_t s, LevelView<T> L, const T* lfac, int mode, const T* f, const T* dinv,
                    const T* x_old, T* x_prev, T* x_new, T* dv, T* scr, T c1, T c2, T c0, const T* fd) {
   if (lfac) {

@@ -229,6 +229,7 @@ __device__ __forceinline__ void smooth_point_pair(const LevelView<T>& L, const T
     st_pair(x_prev, at.c, at.both, row[0] ? xs.v[0][0] : T(0), row[1] ? xs.v[0][1] : T(0));
   st_pair(x_new, at.c, at.both, xn[0], xn[1]);
 }
+
 // Thomas factors of the y-line tridiagonal part of A on the line (i, k), from the
 // rows' SP / CP / NP coefficients (cells without an unknown get the identity):
 // lfac = [a | cp | inv], each n long; den_j = b_j - a_j cp_{j-1}, inv_j = 1/den_j,

@@ -460,7 +460,8 @@ __device__ __forceinline__ double wave_max_all(double v) {
 
 // One panel: columns k .. k + nb - 1 of A (N x N, row-major), one block, R rows per
 // thread with the panel's entries in registers.  Step c picks the pivot, the
-// first largest |A[r][k + c]| over the rows that no earlier column took, and eliminates
+// largest |A[r][k + c]| over the rows that no earlier column took (of equal ones the
+// lowest lane's in the lowest wave: the first row, up to 1024 rows), and eliminates
 // column k + c from every other row of the panel in place: entry (r, k + c) becomes the
 // multiplier of the pivot row.  Rows stay where they are (the column that takes row p is
 // kept in q[p], the row column c takes in p[c]; q starts at -1).  At the end T
