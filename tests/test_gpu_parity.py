@@ -36,6 +36,28 @@ def affine_case(nx=10, ny=9, nz=8, seed=0):
     return cases.Case(name="affine", nx=nx, ny=ny, nz=nz, per=(0, 0, 0), bctype=(0,) * 6, immersed=0, fields=f)
 
 
+def sheared_case(nx, ny, nz, per, seed=0):
+    """The affine map of affine_case on any periodicity, with a sphere in the middle and a
+    random flux field that carries nothing through the walls."""
+    M = np.array([[1.0, 0.35, -0.2], [0.15, 0.8, 0.1], [-0.25, 0.3, 1.2]])
+    P = np.stack(np.meshgrid(np.arange(nx + 1) / nx, np.arange(ny + 1) / ny, np.arange(nz + 1) / nz,
+                             indexing="ij"), -1).transpose(2, 1, 0, 3)
+    f = cases.form_metrics(cases.dmda_coords(P @ M.T), per)
+    centre = cases.cell_centres(cases.dmda_coords(P))
+    nv = cases.classify_nvert(cases.interior_only(cases.inside_sphere(centre, (0.45, 0.55, 0.5), 0.2)))
+    cases.periodic_fill(nv, per)
+    f["nvert"] = nv
+    u = np.zeros(nv.shape + (3,))
+    u[1:-1, 1:-1, 1:-1] = np.random.default_rng(seed).standard_normal((nz, ny, nx, 3))
+    for a in range(3):
+        if not per[a]:
+            np.moveaxis(u[..., a], 2 - a, 0)[-2] = 0.0
+    cases.set_periodic_flux_ghosts(u, per)
+    f["ucont"] = u
+    return cases.Case(name=f"sheared{nx}x{ny}x{nz}per{''.join(map(str, per))}", nx=nx, ny=ny, nz=nz, per=per,
+                      bctype=(0,) * 6, immersed=1, fields=f)
+
+
 def _sphere_immersed0():
     c = cases.hill_case(24, 16, 16, h=0.3, sphere=(0.6, 0.75, 0.0, 0.3), seed=1)
     c.immersed = 0
@@ -751,10 +773,20 @@ def test_pair_walk(E, torch_cuda, dims):
     shares none of that code: |b - A Phi| <= 1e-11 |b| from a true residual of 1e-12 |b|,
     with the rounding of a 19-term row on top (the two forms' rows differ by at most
     38 eps |A| |Phi|, far below 1e-11 |b| at these sizes)."""
-    torch = torch_cuda
     nx, ny, nz = dims
-    c = (cases.hill_case(nx, ny, nz, h=0.2, beta=1.5, sphere=(0.6, 0.9, 0.0, 0.25), seed=8) if nx > 100 and nz > 3
-         else cases.channel_case(nx, ny, nz, beta=1.5, seed=8))
+    _pair_walk(E, torch_cuda,
+               cases.hill_case(nx, ny, nz, h=0.2, beta=1.5, sphere=(0.6, 0.9, 0.0, 0.25), seed=8)
+               if nx > 100 and nz > 3 else cases.channel_case(nx, ny, nz, beta=1.5, seed=8))
+
+
+@pytest.mark.parametrize("per", [(0, 0, 0), (1, 1, 1), (0, 1, 0), (0, 0, 1), (1, 1, 0)])
+def test_pair_walk_on_other_topologies(E, torch_cuda, per):
+    """test_pair_walk with walls in i and k and with periodic j, on a sheared grid with a
+    sphere: the wrapped columns and rows of the pairs and the walls' one-sided rows."""
+    _pair_walk(E, torch_cuda, sheared_case(65, 34, 33, per, seed=5))
+
+
+def _pair_walk(E, torch, c):
     print(f"pair walk: {c.name}", flush=True)
     A = O.Assembled(c, drop=False)
     for precision in (0, 1):
