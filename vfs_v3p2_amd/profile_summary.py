@@ -20,8 +20,8 @@ dispatch (and per wave, given SQ_WAVES) of every counter those runs collected.
 Traffic mode reads one FETCH_SIZE and one WRITE_SIZE pass (KiB per dispatch),
 scales each by what the same counter reads for the 1 GiB device copy kernel
 (k_copy16: 1 GiB read, 1 GiB written), and prints HBM-side bytes per launch and
-per cell for every kernel whose grid covers N cells, plus a machine-readable
-line for the finest FP32 smoother sweep.
+per cell for every kernel whose grid covers N cells at one or two per thread, plus a
+machine-readable line for the finest FP32 smoother sweep.
 """
 from __future__ import annotations
 
@@ -84,7 +84,8 @@ def traffic(fetch_csv, write_csv, cells, top):
           f"-> scale {fs:.4f}; WRITE_SIZE reads {W[COPY][0]:.0f} KiB -> scale {ws:.4f}\n")
     print("| kernel | grid | dispatches | fetched MB | written MB | B/cell |")
     print("|---|---|---|---|---|---|")
-    keys = sorted((k for k in F if k[1] == cells), key=lambda k: -(F[k][0] * fs + W.get(k, (0, 0))[0] * ws))
+    grids = (cells, -(-cells // 512) * 256)  # a thread per cell, or per pair in 256-thread blocks
+    keys = sorted((k for k in F if k[1] in grids), key=lambda k: -(F[k][0] * fs + W.get(k, (0, 0))[0] * ws))
     for k in keys[:top]:
         f = F[k][0] * 1024 * fs
         w = W.get(k, (0.0, 0))[0] * 1024 * ws
