@@ -243,11 +243,12 @@ def test_results_do_not_depend_on_the_members_beside(E, torch_cuda, precision, s
     """A member's Phi, Ucont, P and Ucat are the same bits in a batch of one and beside
     members that take the batch across every bound of the kernel choices: 65536 cells, and
     4096, 8192 and 16384 y-lines.  Members: narrow levels below 65536 cells, one above;
-    lines of up to 64, 128, 192, 224 and 256 rows with few lines each, one with 5184 lines
-    of 136 rows and one with 16384 lines.  Six iterations, whether converged or not."""
+    lines of up to 64, 128, 192, 224 and 256 rows with few lines each, one with 1296 lines
+    of 230 rows, one with 5184 of 136 rows and one with 16384.  Six iterations, whether
+    converged or not."""
     torch = torch_cuda
-    dims = [(24, 20, 28), (40, 40, 40), (20, 100, 24), (20, 140, 24), (20, 200, 24), (20, 240, 24), (72, 136, 72),
-            (128, 66, 128)]
+    dims = [(24, 20, 28), (40, 40, 40), (20, 100, 24), (20, 140, 24), (20, 200, 24), (20, 240, 24), (36, 230, 36),
+            (72, 136, 72), (128, 66, 128)]
     cs = []
     for q, (nx, ny, nz) in enumerate(dims):
         sphere = (0.6, 0.9, 0.0, 0.3) if q % 2 else None

@@ -855,7 +855,7 @@ struct BatchCore {
   static uint32_t line_tiles(const Dims& d) { return (uint32_t)(((size_t)d.nx * d.nz + 255) / 256); }
   static uint32_t seg_line_tiles(const Dims& d, int layout) {
     size_t lanes = 1;
-    with_line_layout<T>(layout, [&](auto y) { lanes = decltype(y)::LANES; });
+    with_line_layout<T, true>(layout, [&](auto y) { lanes = decltype(y)::LANES; });
     return (uint32_t)(((size_t)d.nx * d.nz + lanes - 1) / lanes);
   }
   static bool seg_lines(const Dims& d) { return line_seg_fits<T>(d); }
@@ -928,7 +928,7 @@ struct BatchCore {
         it.tx = (uint32_t)(L.d.nx + 63) / 64;
         it.ty = 0;
         if (seg_lines(L.d)) {
-          const int lay = line_layout<T>(L.d.ny, (size_t)L.d.nx * L.d.nz, lines);
+          const int lay = batch_line_layout<T>(L.d.ny, (size_t)L.d.nx * L.d.nz, lines);
           smode = mode;
           sg[lay].push_back(it);
           nsg[lay].push_back(seg_line_tiles(L.d, lay));
@@ -1220,7 +1220,7 @@ struct BatchCore {
                                                            L.nitems, L.total, sd);
         break;
       case K_LSEG:
-        with_line_layout<T>(L.mode >> 3, [&](auto lay) {
+        with_line_layout<T, true>(L.mode >> 3, [&](auto lay) {
           using Y = decltype(lay);
           auto* it = static_cast<const SmoothItem<T>*>(L.items);
           if ((L.mode & 7) == SM_ZERO)

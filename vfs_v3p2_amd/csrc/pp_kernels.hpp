@@ -208,8 +208,7 @@ template <typename T>
 HD inline bool line_seg_fits(const Dims& d) {
   return d.ny <= 256;
 }
-// Block layout of the segmented step for lines of ny rows of a level of `own` lines, in a
-// launch of `all` lines (a batched launch holds its members' levels): an index into
+// Block layout of the segmented step for `lines` lines of ny rows: an index into
 // with_line_layout's layouts.  Few lines take narrow blocks of few waves, so that every CU
 // gets some and a block's barriers cost little; many lines take wide ones, whose 256-byte
 // accesses stream from HBM better.
@@ -221,23 +220,42 @@ HD inline bool line_seg_fits(const Dims& d) {
 // x waves x lanes): 256x150x200 332 / 278 / 285 / 306, 100x200x100 69.3 / - / 82.7 / 80.0,
 // 256x200x128 247 / - / 232 / 237, 128x256x64 65.9 / - / 51.6 / 49.0, 512x256x256 1141 / - /
 // 1119 / 1098.
-// The number of segments per line sets how the line's sweeps round, so it follows from the
-// level's own lines alone; the launch's lines pick among layouts of that many segments (16,
-// or 32 in FP32 layout 4 and FP64 layouts 1 and 4), which give the same bits.  A batched
-// member's results therefore do not depend on the members beside it.
-constexpr int LINE_LAYOUTS = 7;
 template <typename T>
-inline int line_layout(int ny, size_t own, size_t all) {
+inline int line_layout(int ny, size_t lines) {
   if (sizeof(T) == 4) {
-    if (ny <= 64) return all < 8192 ? 0 : 1;
-    if (ny <= 128) return all < 8192 ? 2 : 3;
+    if (ny <= 64) return lines < 8192 ? 0 : 1;
+    if (ny <= 128) return lines < 8192 ? 2 : 3;
+    return lines < 4096 ? 4 : lines < 16384 ? 5 : 6;
+  }
+  if (ny <= 64) return 0;
+  if (ny <= 128) return lines < 8192 ? 1 : 2;
+  if (ny <= 192) return lines < 8192 ? 1 : 3;
+  if (ny <= 224) return lines < 16384 ? 1 : 4;
+  return lines < 8192 ? 1 : 5;
+}
+
+// The same for a level of `own` lines in a batched launch of `all` lines.  The number of
+// segments per line sets how the line's sweeps round, so it follows from the level alone
+// (ny and own): a member's results do not depend on the members beside it.  The launch's
+// lines pick among layouts of that many segments (16; 32 in FP32 layout 4 and FP64 layouts 1
+// and 4), which give the same bits.  FP64 takes 16 where line_layout takes 32 for few lines,
+// because 32 cost groups of small members 8 to 11%: batch of 32 56x96x56 25.0 (32 segments)
+// / 22.4 ms (16), 12 80x110x80 23.9 / 21.7, 16 48x160x48 14.6 / 13.4, 16 48x240x48 21.9 /
+// 20.1; alone, 56x96x56 takes 2.46 ms either way (layout 6 for few lines), 72x160x72 3.93 /
+// 3.70, 72x240x72 5.19 / 4.90.  Below 1024 lines, lines of more than 128 rows keep 32 (step
+// of 32x150x32 16.4 / 18.6 us, 24x230x24 24.1 / 28.8).
+constexpr int LINE_LAYOUTS = 8;
+template <typename T>
+inline int batch_line_layout(int ny, size_t own, size_t all) {
+  if (sizeof(T) == 4) {
+    if (ny <= 128) return line_layout<T>(ny, all);
     return own < 4096 ? 4 : all < 16384 ? 5 : 6;
   }
   if (ny <= 64) return 0;
-  if (ny <= 128) return own < 8192 ? 1 : 2;
-  if (ny <= 192) return own < 8192 ? 1 : 3;
+  if (ny <= 128) return all < 8192 ? 6 : 2;
+  if (ny <= 192) return own < 1024 ? 1 : 3;
   if (ny <= 224) return all < 16384 ? 1 : 4;
-  return own < 8192 ? 1 : 5;
+  return own < 1024 ? 1 : all < 8192 ? 7 : 5;
 }
 
 // Chebyshev smoothing launch modes (see smooth_point_cell); SM_POWER is one step

@@ -169,8 +169,8 @@ template <int LM_, int W_, int LANES_, int KEEP_>
 struct LineLayout {
   static constexpr int LM = LM_, W = W_, LANES = LANES_, S = W_ * 64 / LANES_, KEEP = KEEP_;
 };
-// Calls fn with layout y's LineLayout (see line_layout)
-template <typename T, typename F>
+// Calls fn with layout y's LineLayout (see line_layout, and batch_line_layout for BATCHED)
+template <typename T, bool BATCHED = false, typename F>
 inline void with_line_layout(int y, F&& fn) {
   if constexpr (std::is_same<T, float>::value) {
     switch (y) {
@@ -183,6 +183,10 @@ inline void with_line_layout(int y, F&& fn) {
       default: fn(LineLayout<16, 16, 64, 1>{});
     }
   } else {
+    if constexpr (BATCHED) {
+      if (y == 6) return fn(LineLayout<8, 4, 16, 0>{});
+      if (y == 7) return fn(LineLayout<16, 4, 16, 0>{});
+    }
     switch (y) {
       case 0: fn(LineLayout<4, 4, 16, 2>{}); break;
       case 1: fn(LineLayout<8, 8, 16, 0>{}); break;

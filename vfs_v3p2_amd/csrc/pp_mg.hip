@@ -615,7 +615,7 @@ template <typename T>
 static void launch_line_step(hipStream_t s, const LevelView<T>& L, int mode, const T* f, const T* lfac,
                              const T* x_old, const T* x_prev, T* x_new, T c1, T c2) {
   const size_t lines = (size_t)L.d.nx * L.d.nz;
-  with_line_layout<T>(line_layout<T>(L.d.ny, lines, lines), [&](auto lay) {
+  with_line_layout<T>(line_layout<T>(L.d.ny, lines), [&](auto lay) {
     using Y = decltype(lay);
     const dim3 gr((unsigned)((lines + Y::LANES - 1) / Y::LANES)), bl(64, Y::W);
     if (mode == LS_ZERO)
@@ -631,7 +631,7 @@ template <typename T>
 double line_step_coef_bytes(const Dims& d) {
   int keep = 0;
   const size_t lines = (size_t)d.nx * d.nz;
-  with_line_layout<T>(line_layout<T>(d.ny, lines, lines), [&](auto lay) { keep = decltype(lay)::KEEP; });
+  with_line_layout<T>(line_layout<T>(d.ny, lines), [&](auto lay) { keep = decltype(lay)::KEEP; });
   // FP32: the three records, and cp where it is read after the walk; FP64: coefficients,
   // class byte and 1 / den, and a and cp where they are read after the walk
   if (sizeof(T) == 4) return 24 + (keep < 2 ? 4 : 0) + (keep < 1 ? 4 : 0);
